@@ -19,7 +19,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 HOST_SRCS = ["host/refelem.cpp", "host/mesh.cpp", "host/datain.cpp"]
-HIP_SRCS = ["solver.hip", "ws_dirichlet.hip"]
+HIP_SRCS = ["solver.hip", "ws_dirichlet.hip", "cols_euler_low.hip", "cols_euler_high.hip", "cols_advection.hip"]
 
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
@@ -77,7 +77,7 @@ def build(verbose=True):
         o = os.path.join(BUILD, os.path.basename(s) + ".o")
         jobs.append([HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, s), "-o", o])
         objs.append(o)
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
         list(ex.map(lambda c: _run(c, verbose), jobs))
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)

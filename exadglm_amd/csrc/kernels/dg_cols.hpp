@@ -1,0 +1,708 @@
+// FP64 stage kernel on MFMA with packed columns (gfx950): Euler and advection,
+// every order, any mesh size.
+//
+// The stage contraction  rhs[v][e][i] = sum_k A[i][k] B[k][(v, e)]  (update_rhs,
+// dim3/src/cpp/euler_dglm.cpp:254-302; A = [WDr|WDs|WDt|-LIFT]) has as columns
+// every (variable, element) pair.  A workgroup takes EB elements, packs their
+// EB*NV columns into CT tiles of 16, and goes through
+//   1. node values -> LDS, with the primitives the volume fluxes are formed
+//      from (pressure and contravariant velocity; for advection the three
+//      contravariant fluxes); the gathers of the exterior traces are issued
+//      and stay in registers;
+//   2. the volume k-steps (three directions of four nodes at a time), whose
+//      B-fragments are formed in registers, f_d = c V_d + p g_d,v-1;
+//   3. the surface flux of all variables at every face node, once, into the
+//      LDS the primitives held;
+//   4. the surface k-steps and the LSRK update.
+//
+// Rows: sixteen at a time on v_mfma_f64_16x16x4f64, what is left of Np in
+// units of four on v_mfma_f64_4x4x4f64 with the unit's A in all four blocks,
+// which then is a 4 x 16 tile: the same flops per cycle (64.2 against 68.1
+// TF/s measured, 256 CUs) and the same B-fragment, so Np rows cost ceil(Np/4)
+// units and not 4 ceil(Np/16).  The operator is streamed from the L2 in the
+// order each wave uses it.
+//
+// What the layout is for: every vector memory instruction of a wave takes the
+// CU's L1 at least 16 cycles (64 where each lane is on a line of its own), and
+// no VALU instruction overlaps an FP64 MFMA.  Hence 16-byte operator loads
+// that serve a whole block of k-steps, the new state written through LDS in
+// memory order, and as many columns per operator load as the LDS holds.
+#pragma once
+#include <type_traits>
+
+#include "cols_ops.h"
+#include "dg_mfma.hpp"
+
+namespace dglm {
+
+// Rows of one wave: nt tiles from tile0 with every column tile; one column
+// tile (c0) of tile xt (-1: none); nq units of four rows from unit q0 with
+// every column tile.
+struct ColRole {
+  int tile0, nt, xt, c0, q0, nq;
+  constexpr int na() const { return nt + (xt >= 0 ? 1 : 0) + nq; }
+  constexpr bool same(const ColRole &o) const { return nt == o.nt && (xt >= 0) == (o.xt >= 0) && nq == o.nq; }
+};
+
+template <int NW>
+struct ColRoles {
+  ColRole r[NW];
+};
+
+// Deal the G row units (G / 4 tiles, G % 4 single units) and CT column tiles
+// to NW waves: equal numbers of tiles first; of the tiles left over, whole
+// ones while there are more (tile, column) items than waves, then one item to
+// a wave; each single unit to the wave with the least work.
+template <int G, int CT, int NW>
+constexpr ColRoles<NW> cols_roles() {
+  ColRoles<NW> R{};
+  const int tiles = G / 4, base = tiles / NW, rt = tiles % NW;
+  int n = CT == 1 ? rt : 0;
+  while ((rt - n) * CT > NW - n) n++;
+  int load[NW] = {}, t = 0;
+  for (int w = 0; w < NW; w++) {
+    R.r[w] = ColRole{t, base + (w < n ? 1 : 0), -1, 0, 4 * tiles, 0};
+    t += R.r[w].nt;
+    load[w] = 4 * CT * R.r[w].nt;
+  }
+  for (int i = 0; i < (rt - n) * CT; i++) {
+    R.r[n + i].xt = t + i / CT;
+    R.r[n + i].c0 = i % CT;
+    load[n + i] += 4;
+  }
+  for (int q = 4 * tiles; q < G; q++) {
+    int b = NW - 1;
+    for (int w = NW - 1; w >= 0; w--)
+      if (load[w] + (R.r[w].nq ? -1 : 0) < load[b] + (R.r[b].nq ? -1 : 0)) b = w;
+    // a wave's units are consecutive: the rest of the units of a wave that has some
+    if (R.r[b].nq && R.r[b].q0 + R.r[b].nq != q) {
+      b = 0;
+      for (int w = 0; w < NW; w++)
+        if (R.r[w].nq && R.r[w].q0 + R.r[w].nq == q) b = w;
+    }
+    if (!R.r[b].nq) R.r[b].q0 = q;
+    R.r[b].nq++;
+    load[b] += CT;
+  }
+  return R;
+}
+
+template <int N, int PHYS, int EB_, int NW_>
+struct ColShape {
+  using O = Ord<N>;
+  static constexpr int NV = NVar<PHYS>::value;
+  static constexpr int Np = O::Np, Nfp = O::Nfp, NFF = O::NFF;
+  static constexpr int G = (Np + 3) / 4;  // groups of four nodes: blocks of three k-steps, and row units
+  static constexpr int KSS = Nfp;         // surface k-steps
+  static constexpr int SB = (KSS + 2) / 3, SLAST = KSS - 3 * (SB - 1);  // their blocks; k-steps of the last one
+  static constexpr int NBLK = G + SB;
+  static constexpr int NS = 4 * (G | 1);  // element stride of the node arrays: an odd number of groups of four, so
+                                          // that the 16 columns x 4 nodes of a fragment read fall on the 32 LDS
+                                          // bank pairs twice each (nodes Np..4G-1 are zero)
+  static constexpr int EB = EB_, NW = NW_, NT = 64 * NW;
+  static constexpr int NC = EB * NV, CT = (NC + 15) / 16;
+  static constexpr int CS = 16 * CT + 1;                 // row stride of the surface fluxes (odd: a wave writes
+                                                         // consecutive face nodes of one column)
+  static constexpr int NA = PHYS == PHYS_EULER ? 4 : 3;  // volume arrays: V_0..2 and p, or f_0..2
+  static constexpr int VOL = NA * EB * NS, SUR = NFF * CS, OUT = NC * NS;
+  static constexpr int X = VOL > SUR ? (VOL > OUT ? VOL : OUT) : (SUR > OUT ? SUR : OUT);
+  static constexpr ColRoles<NW> roles = cols_roles<G, CT, NW>();
+  // operator stream of wave w: blocks of 3 k-steps, each lane's 3 na values of a
+  // block as 16-byte pairs [pair][lane][2] and, where 3 na is odd, [lane] doubles
+  static constexpr size_t stream(int w) {
+    size_t o = 0;
+    for (int i = 0; i < w; i++) o += (size_t)NBLK * 3 * roles.r[i].na() * 64;
+    return o;
+  }
+};
+
+// Host side: the operator streams of all waves (ColShape::stream(NW) doubles).
+// Value x of a lane in a block is k-step x / na, row set x % na: its tiles,
+// then xt, then its units.  A tile's lane l holds tile row 4 (l % 4) + (l / 4) % 4,
+// so that a lane's four results are consecutive rows; a unit's lane l holds
+// row l % 4; both column l / 16 of the k-step.
+template <class S>
+inline void cols_arrange(const double *opT /*[KD][Np]*/, double *out) {
+  for (int w = 0; w < S::NW; w++) {
+    const ColRole r = S::roles.r[w];
+    const int na = r.na();
+    double *o = out + S::stream(w);
+    for (int b = 0; b < S::NBLK; b++)
+      for (int x = 0; x < 3 * na; x++)
+        for (int l = 0; l < 64; l++) {
+          const int d = x / na, i = x % na, kk = l >> 4;
+          int row, k;
+          if (i < r.nt)
+            row = 16 * (r.tile0 + i) + 4 * (l & 3) + ((l >> 2) & 3);
+          else if (i == r.nt && r.xt >= 0)
+            row = 16 * r.xt + 4 * (l & 3) + ((l >> 2) & 3);
+          else
+            row = 4 * (r.q0 + i - r.nt - (r.xt >= 0 ? 1 : 0)) + (l & 3);
+          if (b < S::G) {
+            const int j = 4 * b + kk;
+            k = j < S::Np ? d * S::Np + j : -1;
+          } else {
+            const int m = 4 * (3 * (b - S::G) + d) + kk;
+            k = m < S::NFF ? 3 * S::Np + m : -1;
+          }
+          const size_t at = x < 3 * na / 2 * 2 ? ((size_t)(x / 2) * 64 + l) * 2 + (x & 1) : (size_t)(3 * na - 1) * 64 + l;
+          o[(size_t)b * 3 * na * 64 + at] = row < S::Np && k >= 0 ? opT[(size_t)k * S::Np + row] : 0.0;
+        }
+  }
+}
+
+// Two doubles at an 8-byte aligned address: one 16-byte memory instruction.
+typedef double f64x2a8 __attribute__((ext_vector_type(2), aligned(8)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+// Surface flux of the five variables times Fscale at one face node, g = (nx,
+// ny, nz, Fscale): LM, whose face state ub is the mean of the traces (on a
+// Dirichlet face the prescribed state uP), or Rusanov.
+__device__ inline void cols_surface_flux5(const double uM[5], const double uP[5], bool dirichlet, const double *g,
+                                          double tau, int flux, double gamma, double fl[5]) {
+  auto normal = [&](const double U[5], double &lam, double F[5]) {
+    const double inv = rcp_refined(U[0]);
+    const double p = (gamma - 1.0) * (U[4] - 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) * inv);
+    const double mn = g[0] * U[1] + g[1] * U[2] + g[2] * U[3], vn = mn * inv;
+    lam = flux == 1 ? fabs(vn) + sqrt_refined(fabs(gamma * p * inv)) : 0.0;
+    F[0] = mn;
+    F[1] = U[1] * vn + g[0] * p;
+    F[2] = U[2] * vn + g[1] * p;
+    F[3] = U[3] * vn + g[2] * p;
+    F[4] = (U[4] + p) * vn;
+  };
+  double lm;
+  if (flux == 1) {
+    double fm[5], fp[5], lp;
+    normal(uM, lm, fm);
+    normal(uP, lp, fp);
+    const double lam = fmax(lm, lp);
+#pragma unroll
+    for (int v = 0; v < 5; v++) fl[v] = (0.5 * (fm[v] + fp[v]) + 0.5 * lam * (uM[v] - uP[v])) * g[3];
+  } else {
+    double ub[5], nF[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) ub[v] = dirichlet ? uP[v] : 0.5 * (uM[v] + uP[v]);
+    normal(ub, lm, nF);
+#pragma unroll
+    for (int v = 0; v < 5; v++) fl[v] = (nF[v] - tau * (ub[v] - uM[v])) * g[3];
+  }
+}
+
+// Workgroup barrier over LDS: waits for this wave's LDS operations only, so
+// that the gathers, the LSRK registers and the stores stay in flight across it
+// (nothing in a launch reads global memory that the launch writes).
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A lane's operator values of one block.
+template <int NA>
+struct ColA {
+  f64x2 p[3 * NA / 2 > 0 ? 3 * NA / 2 : 1];
+  double o;
+  __device__ inline void load(const double *__restrict__ b, int lane) {
+#pragma unroll
+    for (int i = 0; i < 3 * NA / 2; i++) p[i] = *reinterpret_cast<const f64x2 *>(b + 128 * i + 2 * lane);
+    if constexpr (NA % 2) o = b[(3 * NA - 1) * 64 + lane];
+  }
+  __device__ inline double at(int x) const { return NA % 2 && x == 3 * NA - 1 ? o : p[x / 2][x % 2]; }
+};
+
+// Calls body with wave w's role: one instantiation for each distinct shape.
+template <class S, int I>
+struct ColRoleAt {
+  static constexpr ColRole value = S::roles.r[I];
+};
+template <class S, int I>
+constexpr bool cols_first() {
+  for (int j = 0; j < I; j++)
+    if (S::roles.r[j].same(S::roles.r[I])) return false;
+  return true;
+}
+template <class S, int I, class F>
+__device__ inline void cols_dispatch(int w, F &body) {
+  if constexpr (I < S::NW) {
+    if constexpr (cols_first<S, I>()) {
+      bool mine = false;
+      size_t stream = 0;
+      int tile0 = 0, xt = 0, c0 = 0, q0 = 0;
+#pragma unroll
+      for (int j = I; j < S::NW; j++)
+        if (w == j && S::roles.r[j].same(S::roles.r[I])) {
+          mine = true;
+          stream = S::stream(j);
+          tile0 = S::roles.r[j].tile0;
+          xt = S::roles.r[j].xt;
+          c0 = S::roles.r[j].c0;
+          q0 = S::roles.r[j].q0;
+        }
+      if (mine) {
+        body(ColRoleAt<S, I>{}, stream, tile0, xt, c0, q0);
+        return;
+      }
+    }
+    cols_dispatch<S, I + 1>(w, body);
+  }
+}
+
+//   MODE 0: LSRK update; MODE 1: write the RHS only.
+template <int N, int PHYS, int EB, int NW, int MODE>
+__global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, const double *__restrict__ afrag,
+                                                                  const int *__restrict__ order, int nbatch) {
+  using S = ColShape<N, PHYS, EB, NW>;
+  constexpr int Np = S::Np, Nfp = S::Nfp, NFF = S::NFF, G = S::G, NS = S::NS, NT = S::NT, NV = S::NV;
+  constexpr int NC = S::NC, CT = S::CT, CS = S::CS;
+  constexpr bool EUL = PHYS == PHYS_EULER;
+  constexpr int VW = Np % 2 == 0 ? 2 : 1;  // nodes a thread takes at a time
+  typedef typename std::conditional<VW == 2, f64x2a8, double>::type vec;
+  static_assert(4 * EB <= NT, "one face per thread");
+
+  __shared__ __align__(16) double s_u[NV * EB * NS];
+  // volume arrays [V_0, V_1, V_2(, p)][element][node], then the surface
+  // fluxes [face node][column], then the contraction [column][row]
+  __shared__ __align__(16) double s_x[S::X];
+  __shared__ double s_geo[EB * GEO_STRIDE];
+  __shared__ double s_tau[EB * 4];
+  __shared__ int s_conn[EB * 4];
+  __shared__ int s_dm[EB * 4];
+  __shared__ int s_fmx[16 * Nfp];
+
+  // Batch of this workgroup: workgroup i of XCD x (blocks go to the XCDs
+  // round-robin) takes entry i of the x-th eighth of the visiting order, so
+  // neighbouring batches share an L2.
+  const int xcd = blockIdx.x & 7;
+  const int slot = (int)((long)nbatch * xcd / 8) + (int)(blockIdx.x >> 3);
+  if (slot >= (int)((long)nbatch * (xcd + 1) / 8)) return;
+  const int e0 = (order ? order[slot] : slot) * EB;
+  const int K = a.K;
+  const size_t KNp = (size_t)K * Np;
+  const int ne = min(EB, K - e0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const size_t n0 = (size_t)e0 * Np;
+
+  if (MODE == 0 && !a.scal->active) {
+    // Past tmax: the stage is the identity on u (k untouched).
+    for (int v = 0; v < NV; v++)
+      for (int i = tid; i < ne * Np; i += NT) a.u_out[v * KNp + n0 + i] = a.u_in[v * KNp + n0 + i];
+    return;
+  }
+  const double dt = MODE == 0 ? a.scal->dt : 0.0;
+
+  // ---- 1. stage in.  Elements past the end of a short batch get a state at
+  // rest and no geometry; their columns are computed and not written ----
+  constexpr int RN = (EB * Np / VW + NT - 1) / NT;  // nodes (or pairs) per thread
+  constexpr int RF = (EB * NFF + NT - 1) / NT;      // face nodes per thread
+  double lam_own = 0.0, lam_nbr = 0.0;
+  if (tid < 4 * EB) {
+    const int c = tid < 4 * ne ? a.conn[(size_t)e0 * 4 + tid] : 0;
+    s_conn[tid] = c;
+    s_dm[tid] = a.dmap && tid < 4 * ne ? a.dmap[(size_t)e0 * 4 + tid] : -1;
+    if (tid < 4 * ne) {
+      lam_own = a.maxv[(size_t)e0 * 4 + tid];
+      lam_nbr = a.maxv[(size_t)conn_nbr(c) * 4 + conn_face(c)];
+    }
+  }
+  vec un[RN][NV], vl[EUL ? 1 : RN][3];
+#pragma unroll
+  for (int r = 0; r < RN; r++) {
+    const int i = (tid + NT * r) * VW;
+    const bool live = i < ne * Np;
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      un[r][v] = vec(EUL && v == 0 ? 1.0 : 0.0);
+      if (live) un[r][v] = *reinterpret_cast<const vec *>(a.u_in + v * KNp + n0 + i);
+    }
+    if constexpr (!EUL) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        vl[r][d] = vec(0.0);
+        if (live) vl[r][d] = *reinterpret_cast<const vec *>(a.vel + d * KNp + n0 + i);
+      }
+    }
+  }
+  for (int i = tid; i < 16 * Nfp; i += NT) s_fmx[i] = a.fmx[i];
+  for (int i = tid; i < EB * GEO_STRIDE; i += NT) s_geo[i] = i < ne * GEO_STRIDE ? a.geo[(size_t)e0 * GEO_STRIDE + i] : 0.0;
+  if constexpr (Np % 4 != 0) {  // nodes Np..4G-1
+    for (int i = tid; i < EB * (4 * G - Np); i += NT) {
+      const int o = i / (4 * G - Np) * NS + Np + i % (4 * G - Np);
+#pragma unroll
+      for (int v = 0; v < NV; v++) s_u[v * EB * NS + o] = 0.0;
+#pragma unroll
+      for (int d = 0; d < S::NA; d++) s_x[d * EB * NS + o] = 0.0;
+    }
+  }
+  lds_barrier();
+
+  // exterior traces (and, for advection, the velocity) at this thread's face
+  // nodes; in flight until phase 3
+  double uP[RF][NV], vf[EUL ? 1 : RF][3];
+#pragma unroll
+  for (int r = 0; r < RF; r++) {
+    const int idx = min(tid + NT * r, EB * NFF - 1), e = idx / NFF, m = idx - e * NFF;
+    const int f = m / Nfp, j = m - f * Nfp;
+    const int c = s_conn[e * 4 + f];
+    const size_t pi = (size_t)conn_nbr(c) * Np + s_fmx[(conn_face(c) * 4 + conn_code(c)) * Nfp + j];
+#pragma unroll
+    for (int v = 0; v < NV; v++) uP[r][v] = a.u_in[v * KNp + pi];
+    if constexpr (!EUL) {
+      const size_t mi = e < ne ? n0 + e * Np + s_fmx[(f * 4 + 3) * Nfp + j] : 0;
+#pragma unroll
+      for (int d = 0; d < 3; d++) vf[r][d] = a.vel[d * KNp + mi];
+    }
+  }
+  if (a.dmap) {  // Dirichlet faces: the prescribed state instead
+#pragma unroll
+    for (int r = 0; r < RF; r++) {
+      const int idx = min(tid + NT * r, EB * NFF - 1), e = idx / NFF, m = idx - e * NFF;
+      const int f = m / Nfp, ds = s_dm[e * 4 + f];
+      if (ds >= 0) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) uP[r][v] = dirichlet_value(a, v, ds, m - f * Nfp, Nfp);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RN; r++) {
+    const int i = (tid + NT * r) * VW;
+    if (i < EB * Np) {
+      const int e = i / Np, o = e * NS + i - e * Np;
+      const double *g = &s_geo[e * GEO_STRIDE];
+      vec V[3];
+      if constexpr (EUL) {
+        vec inv;
+        if constexpr (VW == 2)
+          inv = vec{rcp_refined(un[r][0][0]), rcp_refined(un[r][0][1])};
+        else
+          inv = rcp_refined(un[r][0]);
+        const vec p = (a.gamma - 1.0) *
+                      (un[r][4] - 0.5 * (un[r][1] * un[r][1] + un[r][2] * un[r][2] + un[r][3] * un[r][3]) * inv);
+        const vec vx = un[r][1] * inv, vy = un[r][2] * inv, vz = un[r][3] * inv;
+#pragma unroll
+        for (int d = 0; d < 3; d++) V[d] = g[3 * d] * vx + g[3 * d + 1] * vy + g[3 * d + 2] * vz;
+        *reinterpret_cast<vec *>(&s_x[3 * EB * NS + o]) = p;
+      } else {
+        const vec F = vl[r][0] * un[r][0], H = vl[r][1] * un[r][0], L = vl[r][2] * un[r][0];
+#pragma unroll
+        for (int d = 0; d < 3; d++) V[d] = g[3 * d] * F + g[3 * d + 1] * H + g[3 * d + 2] * L;
+      }
+#pragma unroll
+      for (int d = 0; d < 3; d++) *reinterpret_cast<vec *>(&s_x[d * EB * NS + o]) = V[d];
+#pragma unroll
+      for (int v = 0; v < NV; v++) *reinterpret_cast<vec *>(&s_u[v * EB * NS + o]) = un[r][v];
+    }
+  }
+  if (tid < 4 * EB) s_tau[tid] = 0.25 * (lam_own + lam_nbr) * a.tau_scale;
+  lds_barrier();
+
+  const int kk = lane >> 4, cl = lane & 15;
+  constexpr int RO = (NC * Np / VW + NT - 1) / NT;  // values (or pairs) of the update per thread
+  // value i of the update: variable, offset in its batch of nodes, LDS place
+  auto place = [&](int i, int &v, int &n, int &o) {
+    v = i / (EB * Np);
+    n = i - v * (EB * Np);
+    const int e = n / Np;
+    o = (v * EB + e) * NS + n - e * Np;
+  };
+
+  // phases 2..4 of a wave
+  auto body = [&](auto role_, size_t stream, int tile0, int xt, int c0, int q0) {
+    constexpr ColRole role = decltype(role_)::value;
+    constexpr int T = role.nt, XT = role.xt >= 0 ? 1 : 0, Q = role.nq, NA = role.na();
+    constexpr int T1 = T > 0 ? T : 1, Q1 = Q > 0 ? Q : 1;
+    const double *ap = afrag + stream;
+    f64x4 acc[T1][CT], acx = {0.0, 0.0, 0.0, 0.0};
+    double acq[Q1][CT];
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+#pragma unroll
+      for (int i = 0; i < T1; i++) acc[i][t] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int i = 0; i < Q1; i++) acq[i][t] = 0.0;
+    }
+    // local column tile t is tile (c0 + t) % CT: the extra item's is local 0.
+    // This lane's column of it: (variable cv, element ce), dead ones repeat 0
+    int ct[CT], cv[CT], ce[CT];
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+      ct[t] = c0 + t < CT ? c0 + t : c0 + t - CT;
+      const int c = 16 * ct[t] + cl;
+      cv[t] = c < NC ? c / EB : 0;
+      ce[t] = c < NC ? c - cv[t] * EB : 0;
+    }
+    ColA<NA> A[2];
+    auto contract = [&](const ColA<NA> &Ad, const double (&Bd)[3][CT], int n) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        if (d >= n) continue;
+#pragma unroll
+        for (int i = 0; i < T; i++)
+#pragma unroll
+          for (int t = 0; t < CT; t++)
+            acc[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ad.at(d * NA + i), Bd[d][t], acc[i][t], 0, 0, 0);
+        if constexpr (XT) acx = __builtin_amdgcn_mfma_f64_16x16x4f64(Ad.at(d * NA + T), Bd[d][0], acx, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < Q; i++)
+#pragma unroll
+          for (int t = 0; t < CT; t++)
+            acq[i][t] = __builtin_amdgcn_mfma_f64_4x4x4f64(Ad.at(d * NA + T + XT + i), Bd[d][t], acq[i][t], 0, 0, 0);
+      }
+    };
+
+    // ---- 2. volume k-steps ----
+    // A block's operator values and node values are loaded while the block
+    // before it is contracted; the fences keep the compiler from sinking the
+    // loads to their uses.
+    if constexpr (NA > 0) {
+      A[0].load(ap, lane);
+      int oe[CT], ou[CT];
+      double gv[CT][3], fe[CT];
+#pragma unroll
+      for (int t = 0; t < CT; t++) {
+        oe[t] = ce[t] * NS + kk;
+        ou[t] = cv[t] * EB * NS + oe[t];
+        if constexpr (EUL) {
+          const bool mom = cv[t] >= 1 && cv[t] <= 3;
+#pragma unroll
+          for (int d = 0; d < 3; d++) gv[t][d] = mom ? s_geo[ce[t] * GEO_STRIDE + 3 * d + (mom ? cv[t] - 1 : 0)] : 0.0;
+          fe[t] = cv[t] == 4 ? 1.0 : 0.0;
+        }
+      }
+      constexpr int NR = EUL ? 5 : 3;  // node values of a column
+      double R[CT][NR], B[3][CT];
+      auto read = [&](int g) {
+#pragma unroll
+        for (int t = 0; t < CT; t++) {
+#pragma unroll
+          for (int d = 0; d < 3; d++) R[t][d] = s_x[d * EB * NS + oe[t] + 4 * g];
+          if constexpr (EUL) {
+            R[t][3] = s_x[3 * EB * NS + oe[t] + 4 * g];
+            R[t][4] = s_u[ou[t] + 4 * g];
+          }
+        }
+      };
+      auto form = [&]() {
+#pragma unroll
+        for (int t = 0; t < CT; t++) {
+          if constexpr (EUL) {
+            const double c = R[t][4] + fe[t] * R[t][3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) B[d][t] = c * R[t][d] + R[t][3] * gv[t][d];
+          } else {
+#pragma unroll
+            for (int d = 0; d < 3; d++) B[d][t] = R[t][d];
+          }
+        }
+      };
+      auto step = [&](int g, int cur) {
+        A[cur ^ 1].load(ap + (size_t)(g + 1) * (3 * NA * 64), lane);
+        form();
+        read(g + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        contract(A[cur], B, 3);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      read(0);
+      constexpr int G2 = (G - 1) / 2 * 2;
+#pragma unroll 1
+      for (int g = 0; g < G2; g += 2) {
+        step(g, 0);
+        step(g + 1, 1);
+      }
+      if constexpr (G2 < G - 1) step(G2, 0);
+      form();
+      contract(A[(G - 1) & 1], B, 3);
+    }
+    lds_barrier();  // the volume arrays are read: their LDS takes the surface fluxes
+
+    // ---- 3. surface fluxes ----
+#pragma unroll
+    for (int r = 0; r < RF; r++) {
+      const int i = tid + NT * r, idx = min(i, EB * NFF - 1), e = idx / NFF, m = idx - e * NFF;
+      const int f = m / Nfp, j = m - f * Nfp;
+      const int o = e * NS + s_fmx[(f * 4 + 3) * Nfp + j];
+      const double *g = &s_geo[e * GEO_STRIDE + 9 + f * 4];
+      const double tau = s_tau[e * 4 + f];
+      const bool dir = a.dmap && s_dm[e * 4 + f] >= 0;
+      double fl[NV];
+      if constexpr (EUL) {
+        double uM[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++) uM[v] = s_u[v * EB * NS + o];
+        cols_surface_flux5(uM, uP[r], dir, g, tau, a.flux, a.gamma, fl);
+      } else {
+        const double uM = s_u[o], up = uP[r][0];
+        const double ub = dir && a.flux != 1 ? up : 0.5 * (uM + up);
+        if (a.flux == 1) {
+          const double vn = g[0] * vf[r][0] + g[1] * vf[r][1] + g[2] * vf[r][2];
+          fl[0] = (vn * ub + 0.5 * fabs(vn) * (uM - up)) * g[3];
+        } else {
+          const double nF = g[0] * (vf[r][0] * ub) + g[1] * (vf[r][1] * ub) + g[2] * (vf[r][2] * ub);
+          fl[0] = (nF - tau * (ub - uM)) * g[3];
+        }
+      }
+      if (i < EB * NFF) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) s_x[m * CS + v * EB + e] = fl[v];
+      }
+    }
+    lds_barrier();
+
+    // ---- 4. surface k-steps; the LSRK registers arrive meanwhile ----
+    vec kr[RO];
+    if (MODE == 0) {
+#pragma unroll
+      for (int r = 0; r < RO; r++) {
+        const int i = (tid + NT * r) * VW;
+        int v, n, o;
+        place(min(i, NC * Np - VW), v, n, o);
+        kr[r] = vec(0.0);
+        if (n < ne * Np) kr[r] = *reinterpret_cast<const vec *>(a.k + v * KNp + n0 + n);
+      }
+    }
+    if constexpr (NA > 0) {
+      constexpr int SB = S::SB;
+      const double *as = ap + (size_t)G * (3 * NA * 64);
+      double B[2][3][CT];
+      auto read = [&](double (&Bd)[3][CT], int s, int n) {
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+          if (d < n)
+#pragma unroll
+            for (int t = 0; t < CT; t++) Bd[d][t] = s_x[(4 * (3 * s + d) + kk) * CS + 16 * ct[t] + cl];
+      };
+      auto step = [&](int s, int cur, int n) {  // n: k-steps of block s + 1
+        A[cur ^ 1].load(as + (size_t)(s + 1) * (3 * NA * 64), lane);
+        read(B[cur ^ 1], s + 1, n);
+        __builtin_amdgcn_sched_barrier(0);
+        contract(A[cur], B[cur], 3);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      A[0].load(as, lane);
+      read(B[0], 0, SB > 1 ? 3 : S::SLAST);
+      constexpr int M = SB > 1 ? SB - 2 : 0, M2 = M / 2 * 2;  // steps whose next block is full
+#pragma unroll 1
+      for (int s = 0; s < M2; s += 2) {
+        step(s, 0, 3);
+        step(s + 1, 1, 3);
+      }
+      if constexpr (M2 < M) step(M2, 0, 3);
+      if constexpr (SB > 1) step(SB - 2, M & 1, S::SLAST);
+      contract(A[(SB - 1) & 1], B[(SB - 1) & 1], S::SLAST);
+    }
+    lds_barrier();  // the surface fluxes are read: their LDS takes the contraction
+    auto out = [&](int t, int row0, const f64x4 &c) {
+      const int col = 16 * ct[t] + cl;
+      if (col < NC) {
+        f64x2 *d = reinterpret_cast<f64x2 *>(&s_x[col * NS + row0 + 4 * kk]);
+        d[0] = f64x2{c[0], c[1]};
+        d[1] = f64x2{c[2], c[3]};
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+#pragma unroll
+      for (int i = 0; i < T; i++) out(t, 16 * (tile0 + i), acc[i][t]);
+#pragma unroll
+      for (int i = 0; i < Q; i++) {
+        const int col = 16 * ct[t] + cl;
+        if (col < NC) s_x[col * NS + 4 * (q0 + i) + kk] = acq[i][t];
+      }
+    }
+    if constexpr (XT) out(0, 16 * xt, acx);
+    lds_barrier();
+
+    // ---- LSRK update, in memory order ----
+#pragma unroll
+    for (int r = 0; r < RO; r++) {
+      const int i = (tid + NT * r) * VW;
+      int v, n, o;
+      place(min(i, NC * Np - VW), v, n, o);
+      if (i < NC * Np && n < ne * Np) {
+        const size_t gi = v * KNp + n0 + n;
+        const vec rhs = *reinterpret_cast<const vec *>(&s_x[o]);
+        if (MODE == 1) {
+          *reinterpret_cast<vec *>(a.rhs + gi) = rhs;
+        } else {
+          const vec kn = a.rka * kr[r] + dt * rhs;
+          *reinterpret_cast<vec *>(a.k + gi) = kn;
+          *reinterpret_cast<vec *>(a.u_out + gi) = *reinterpret_cast<const vec *>(&s_u[o]) + a.rkb * kn;
+        }
+      }
+    }
+  };
+
+  cols_dispatch<S, 0>(w, body);
+}
+
+// Elements per workgroup and waves: a large and a small configuration of each
+// order.  Measured in us per stage (uniform vortex meshes, Rusanov flux;
+// [EB, waves]):
+//   Euler, K =   1296        6000        13182        24576       82944
+//   N = 2   [3,2] 7.0 [9,2] 7.9   10.1  10.9   18.2  15.4   31.1  26.6
+//   N = 3   [3,2] 7.8 [9,2] 10.5  12.4  15.3   24.1  22.9   39.4  39.5
+//   N = 4   [3,4] 9.7 [9,2] 15.9  23.3  27.0   43.9  50.8   77.7  78.1
+//   N = 5   [3,4] 12.1 [12,4] 18.6  35.9  35.4  72.2  78.2  142  129    488  431
+//   N = 6   [6,4] 20.3 [9,4] 23.5  58.6  62.4   128  126    228  225    714  698
+//   N = 7   [6,4] 29.6 [3,4] 29.4  99.8 107     220  229    399  436
+// Few elements per workgroup while the mesh does not fill the GPU (a stage is
+// then one pass of the chain load, gather, flux, contraction, store), many once
+// it does (each operator load then serves more columns); above N = 7 the LDS
+// holds three elements beside a second workgroup.  For advection a column
+// tile is 16 elements, and 32 were slower (N = 4: 84 against 63 us at K =
+// 82,944; N = 5: 73 against 67 at 48,000).
+struct ColConfig {
+  int eb, nw;
+};
+constexpr ColConfig cols_config(int N, int phys, bool small) {
+  if (phys == PHYS_ADV) return {16, N <= 2 ? N : (N <= 4 || (N <= 6 && !small) ? 4 : 8)};
+  switch (N) {
+    case 1:
+      return small ? ColConfig{6, 2} : ColConfig{16, 2};
+    case 2:
+    case 3:
+      return small ? ColConfig{3, 2} : ColConfig{9, 2};
+    case 4:
+      return small ? ColConfig{3, 4} : ColConfig{9, 2};
+    case 5:
+      return small ? ColConfig{3, 4} : ColConfig{12, 4};
+    case 6:
+      return small ? ColConfig{6, 4} : ColConfig{9, 4};
+    case 7:
+      return {6, 4};
+    default:
+      return {3, 4};
+  }
+}
+// Whether a mesh of K elements takes the small configuration: about where the
+// columns above cross (in small batches: eight a CU; at N = 4 thirty-two).
+constexpr bool cols_small(int N, int phys, int K) {
+  const int nb = (K + cols_config(N, phys, true).eb - 1) / cols_config(N, phys, true).eb;
+  return nb <= (phys == PHYS_EULER && N == 4 ? 8192 : 2048);
+}
+
+template <int N, int PHYS, bool SMALL>
+struct ColImpl {
+  static constexpr ColConfig C = cols_config(N, PHYS, SMALL);
+  using S = ColShape<N, PHYS, C.eb, C.nw>;
+  static void fill(const double *opT, std::vector<double> &out) {
+    out.assign(S::stream(S::NW), 0.0);
+    cols_arrange<S>(opT, out.data());
+  }
+  static void launch(int mode, hipStream_t stream, const StageArgs &a, const double *afrag, const int *order) {
+    const int nbatch = (a.K + C.eb - 1) / C.eb;
+    const dim3 grid((nbatch + 7) / 8 * 8), block(S::NT);
+    if (mode == 1)
+      hipLaunchKernelGGL((stage_cols_kernel<N, PHYS, C.eb, C.nw, 1>), grid, block, 0, stream, a, afrag, order, nbatch);
+    else
+      hipLaunchKernelGGL((stage_cols_kernel<N, PHYS, C.eb, C.nw, 0>), grid, block, 0, stream, a, afrag, order, nbatch);
+  }
+};
+
+// The entry points of one translation unit's orders.
+template <int N, int PHYS>
+inline ColOps cols_ops(int K) {
+  if (cols_small(N, PHYS, K)) return {cols_config(N, PHYS, true).eb, ColImpl<N, PHYS, true>::fill, ColImpl<N, PHYS, true>::launch};
+  return {cols_config(N, PHYS, false).eb, ColImpl<N, PHYS, false>::fill, ColImpl<N, PHYS, false>::launch};
+}
+
+}  // namespace dglm

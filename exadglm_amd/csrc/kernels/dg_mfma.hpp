@@ -1,5 +1,7 @@
-// MFMA stage kernel (gfx950): persistent workgroups, operator resident in
-// registers, per-variable flux tiles in LDS, LSRK update as the epilogue.
+// Generic mixed-precision MFMA stage kernel (gfx950): persistent workgroups,
+// operator resident in registers, per-variable flux tiles in LDS, LSRK update
+// as the epilogue.  It runs the modes the fused mixed-precision kernel
+// (dg_mx.hpp) does not: advection, Dirichlet faces, split BF16.
 //
 // The stage contraction  rhs[v][e][i] = sum_k A[i][k] B_v[k][e]  with
 // A = [WDr | WDs | WDt | -LIFT] (Np x KD) and B_v the stacked volume fluxes
@@ -14,9 +16,8 @@
 //   * the D-fragment is consumed in registers by the LSRK update
 //     k = a k + dt rhs, u_out = u_in + b k (FP64 in every precision).
 //
-// Precision modes:
-//   PREC_F64  v_mfma_f64_16x16x4f64; D register r of lane l is row 4r + l/16,
-//             column l%16.
+// Precision modes (PREC_F64 names the v_mfma_f64_16x16x4f64 traits of the other
+// kernels; D register r of lane l is row 4r + l/16, column l%16):
 //   PREC_F32  v_mfma_f32_16x16x4f32 on  B - c, where c is the least-squares
 //             affine fit of B over the nodes of each (element, variable,
 //             block) -- blocks are the three volume directions and the four
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   constexpr int NV = NVar<PHYS>::value;
   constexpr int EB = 16;
   constexpr int NVEL = PHYS == PHYS_ADV ? 3 : 1;
-  constexpr bool OFFS = PREC != PREC_F64;
+  static_assert(PREC != PREC_F64, "FP64 runs in the packed-column kernel");
   constexpr bool BF = PREC == PREC_BF;
   constexpr int KS16 = S::KS16;
 
@@ -311,8 +312,8 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   __shared__ double s_vel[NVEL][PHYS == PHYS_ADV ? EB * Np : 1];
   __shared__ double s_geo[EB * GEO_STRIDE];
   __shared__ double s_tau[EB * 4];
-  __shared__ double s_b64[OFFS ? KDP * EB : 1];    // FP64 flux tile before the fit is removed
-  __shared__ double s_c[OFFS ? NBLK * 4 * EB : 1];  // affine-fit coefficients [block][q][element]
+  __shared__ double s_b64[KDP * EB];     // FP64 flux tile before the fit is removed
+  __shared__ double s_c[NBLK * 4 * EB];  // affine-fit coefficients [block][q][element]
   // fit = [fitV (KD x 4) | fitP (KD x 4) | fitAV (Np x NBLK x 4)]
   const double *fitV = fit, *fitP = fit + 4 * KD, *fitAV = fit + 8 * KD;
   __shared__ int s_conn[EB * 4];
@@ -430,77 +431,66 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
           for (int q = 0; q < 3; q++) vv[q] = s_vel[q < NVEL ? q : 0] + e * Np;
           volume_flux_v<PHYS>(v, uu, vv, j, &s_geo[e * GEO_STRIDE], a.gamma, f0, f1, f2);
         }
-        if constexpr (OFFS) {
-          s_b64[j * EB + e] = f0;
-          s_b64[(Np + j) * EB + e] = f1;
-          s_b64[(2 * Np + j) * EB + e] = f2;
-        } else {
-          s_f[j * EB + e] = f0;
-          s_f[(Np + j) * EB + e] = f1;
-          s_f[(2 * Np + j) * EB + e] = f2;
-        }
+        s_b64[j * EB + e] = f0;
+        s_b64[(Np + j) * EB + e] = f1;
+        s_b64[(2 * Np + j) * EB + e] = f2;
       }
       // ---- B_v tile: LM surface rows (3Np + m) ----
       for (int idx = tid; idx < NFF * EB; idx += NT) {
         const int m = idx >> 4, e = idx & 15;
         double fl = 0.0;
         if (e < ne) fl = lm_flux(v, e, m);
-        if constexpr (OFFS)
-          s_b64[(3 * Np + m) * EB + e] = fl;
-        else
-          s_f[(3 * Np + m) * EB + e] = fl;
+        s_b64[(3 * Np + m) * EB + e] = fl;
       }
       __syncthreads();
-      if constexpr (OFFS) {
-        // least-squares affine fit per (block, element): c_bq = sum_k fitP[k][q] B_k.
-        // Wave w takes blocks w, w + RT, ...; lane (element e, quarter s) sums
-        // rows k0 + s, k0 + s + 4, ... of the block for all four q, and two
-        // shuffles combine the quarters (a fixed order: deterministic).
-        for (int bb = w; bb < NBLK; bb += S::RT) {
-          const int k0 = bb < 3 ? bb * Np : 3 * Np + (bb - 3) * Nfp, k1 = bb < 3 ? k0 + Np : k0 + Nfp;
-          const int e = lane & 15, sq = lane >> 4;
-          double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
-          for (int k = k0 + sq; k < k1; k += 4) {
-            const double bv = s_b64[k * EB + e];
-            const double *pk = &fitP[k * 4];
-            c0 += pk[0] * bv;
-            c1 += pk[1] * bv;
-            c2 += pk[2] * bv;
-            c3 += pk[3] * bv;
-          }
-#pragma unroll
-          for (int o = 16; o <= 32; o <<= 1) {
-            c0 += __shfl_xor(c0, o, 64);
-            c1 += __shfl_xor(c1, o, 64);
-            c2 += __shfl_xor(c2, o, 64);
-            c3 += __shfl_xor(c3, o, 64);
-          }
-          if (sq == 0) {
-            s_c[(bb * 4 + 0) * EB + e] = c0;
-            s_c[(bb * 4 + 1) * EB + e] = c1;
-            s_c[(bb * 4 + 2) * EB + e] = c2;
-            s_c[(bb * 4 + 3) * EB + e] = c3;
-          }
+      // least-squares affine fit per (block, element): c_bq = sum_k fitP[k][q] B_k.
+      // Wave w takes blocks w, w + RT, ...; lane (element e, quarter s) sums
+      // rows k0 + s, k0 + s + 4, ... of the block for all four q, and two
+      // shuffles combine the quarters (a fixed order: deterministic).
+      for (int bb = w; bb < NBLK; bb += S::RT) {
+        const int k0 = bb < 3 ? bb * Np : 3 * Np + (bb - 3) * Nfp, k1 = bb < 3 ? k0 + Np : k0 + Nfp;
+        const int e = lane & 15, sq = lane >> 4;
+        double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
+        for (int k = k0 + sq; k < k1; k += 4) {
+          const double bv = s_b64[k * EB + e];
+          const double *pk = &fitP[k * 4];
+          c0 += pk[0] * bv;
+          c1 += pk[1] * bv;
+          c2 += pk[2] * bv;
+          c3 += pk[3] * bv;
         }
-        __syncthreads();
-        // the remainder B - fit, rounded to the MFMA precision
-        for (int idx = tid; idx < KD * EB; idx += NT) {
-          const int k = idx >> 4, e = idx & 15;
-          const double *cb = &s_c[offset_block(k, Np, Nfp) * 4 * EB + e];
-          const double *V = &fitV[k * 4];
-          const double fv = cb[0] * V[0] + cb[EB] * V[1] + cb[2 * EB] * V[2] + cb[3 * EB] * V[3];
-          if constexpr (BF) {
-            unsigned short h[BF_PIECES];
-            bf16_split(s_b64[idx] - fv, h);
-            const int pos = ((k >> 4) * 4 + ((k >> 2) & 3)) * EB + e;
 #pragma unroll
-            for (int p = 0; p < BF_PIECES; p++) s_fb[p][pos][k & 3] = (short)h[p];
-          } else {
-            s_f[idx] = (T)(s_b64[idx] - fv);
-          }
+        for (int o = 16; o <= 32; o <<= 1) {
+          c0 += __shfl_xor(c0, o, 64);
+          c1 += __shfl_xor(c1, o, 64);
+          c2 += __shfl_xor(c2, o, 64);
+          c3 += __shfl_xor(c3, o, 64);
         }
-        __syncthreads();
+        if (sq == 0) {
+          s_c[(bb * 4 + 0) * EB + e] = c0;
+          s_c[(bb * 4 + 1) * EB + e] = c1;
+          s_c[(bb * 4 + 2) * EB + e] = c2;
+          s_c[(bb * 4 + 3) * EB + e] = c3;
+        }
       }
+      __syncthreads();
+      // the remainder B - fit, rounded to the MFMA precision
+      for (int idx = tid; idx < KD * EB; idx += NT) {
+        const int k = idx >> 4, e = idx & 15;
+        const double *cb = &s_c[offset_block(k, Np, Nfp) * 4 * EB + e];
+        const double *V = &fitV[k * 4];
+        const double fv = cb[0] * V[0] + cb[EB] * V[1] + cb[2 * EB] * V[2] + cb[3 * EB] * V[3];
+        if constexpr (BF) {
+          unsigned short h[BF_PIECES];
+          bf16_split(s_b64[idx] - fv, h);
+          const int pos = ((k >> 4) * 4 + ((k >> 2) & 3)) * EB + e;
+#pragma unroll
+          for (int p = 0; p < BF_PIECES; p++) s_fb[p][pos][k & 3] = (short)h[p];
+        } else {
+          s_f[idx] = (T)(s_b64[idx] - fv);
+        }
+      }
+      __syncthreads();
 
       // ---- contraction on MFMA ----
       typename P::Acc acc = {0, 0, 0, 0}, acl = {0, 0, 0, 0};
@@ -538,12 +528,10 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
           if (i < Np) {
             double rhs = (double)acc[r];
             if (BF) rhs += (double)acl[r];
-            if (OFFS) {
-              // exact FP64 contraction of the fit: sum_b sum_q c_bq (A_b V_b)_q
-              const double *av = &fitAV[(size_t)i * NBLK * 4];
+            // exact FP64 contraction of the fit: sum_b sum_q c_bq (A_b V_b)_q
+            const double *av = &fitAV[(size_t)i * NBLK * 4];
 #pragma unroll
-              for (int bq = 0; bq < NBLK * 4; bq++) rhs += s_c[bq * EB + e] * av[bq];
-            }
+            for (int bq = 0; bq < NBLK * 4; bq++) rhs += s_c[bq * EB + e] * av[bq];
             const size_t gi = v * KNp + (size_t)(e0 + e) * Np + i;
             if (MODE == 1) {
               a.rhs[gi] = rhs;

@@ -23,6 +23,7 @@
 #include "host/datain.h"
 #include "host/mesh.h"
 #include "host/refelem.h"
+#include "kernels/cols_ops.h"
 #include "kernels/dg_fp64.hpp"
 #include "kernels/dg_step.hpp"
 #include "kernels/dg_mfma.hpp"
@@ -85,7 +86,10 @@ struct dglm_ctx {
   int cur = 0;
   int nblk_ws = 0;
   int variant = DGLM_STAGE_AUTO;  // requested stage kernel
-  void *afrag = nullptr;          // operator A-fragments for the MFMA kernel (FP64 or FP32)
+  void *afrag = nullptr;          // operator A-fragments of the mixed-precision MFMA kernel
+  ColOps cols;                    // the packed-column kernel's entry points for this order and mesh size
+  double *afrag_cols = nullptr;   // its operator streams (null: mixed precision)
+  int *cols_order = nullptr;      // its batch visiting order (null: mesh order)
   double *rowsum = nullptr;       // FP64 affine-offset tables of the mixed-precision contraction
   int mfma_grid = 0;              // persistent grid size (0 = not yet sized)
   double *afrag_ws = nullptr;     // operator rows in the warp-specialised kernel's k order
@@ -270,8 +274,15 @@ void launch_wavespeed(dglm_ctx *c, const double *u, double *maxv, double *partia
                      c->geo, c->fmx, maxv, partial, partial_idx, c->p.gamma);
 }
 
-// True when the MFMA stage kernel is built for this order.
+// True when the MFMA stage kernel can be selected for this order (above it the
+// packed-column kernel is the only FP64 kernel and goes by the name SIMPLE).
 inline bool mfma_available(int N) { return N >= 1 && N <= 6; }
+
+// The warp-specialised kernel pipelines over the 16-element batches of a
+// persistent workgroup; below this many elements (five batches for each of 256
+// CUs) the packed-column kernel is faster at N = 4 (K = 11,520: 37 against 44
+// us per stage; 16,464: 54 and 60; 24,576: 77 and 74; 48,000: 140 and 127).
+constexpr int WS_MIN_ELEMS = 16 * 5 * 256;
 
 // True when the warp-specialised kernel exists for this order.
 inline bool ws_built(int N) {
@@ -286,20 +297,23 @@ inline bool ws_built(int N) {
 }
 
 // The stage kernel that runs: the request where it exists, else the best
-// available: the warp-specialised kernel (FP64, and DGLM_FP32 at N = 3, 4),
-// else the fused mixed-precision kernel (DGLM_FP32 Euler, N <= 6), else the
-// generic MFMA kernel, else the LDS-staged one.
+// available.  FP64: the packed-column kernel (MFMA; SIMPLE above N = 6), but at
+// N = 4 on large Euler meshes the warp-specialised one (at N = 3 the packed
+// columns are faster at every size: K = 1296: 7.8 against 14.6 us per stage,
+// 24,576: 39 and 48, 384,000: 571 and 603).  DGLM_FP32: the warp-specialised
+// kernel at N = 3, 4, else the fused mixed-precision kernel (Euler), else the
+// generic MFMA kernel.
 int stage_kind(const dglm_ctx *c) {
-  const bool ws = c->afrag_ws != nullptr, mf = mfma_available(c->p.N) && c->afrag != nullptr;
-  if (c->variant == DGLM_STAGE_SIMPLE && c->p.precision == DGLM_FP64) return DGLM_STAGE_SIMPLE;
+  const bool ws = c->afrag_ws != nullptr, fp64 = c->p.precision == DGLM_FP64;
+  const bool mf = mfma_available(c->p.N) && (fp64 || c->afrag != nullptr);
+  if (c->variant == DGLM_STAGE_SIMPLE && fp64) return DGLM_STAGE_SIMPLE;
   if (c->variant == DGLM_STAGE_MFMA && mf) return DGLM_STAGE_MFMA;
   if (c->variant == DGLM_STAGE_MFMA_MX && c->mx_tab) return DGLM_STAGE_MFMA_MX;
-  if (ws) return DGLM_STAGE_MFMA_WS;
+  if (ws && (c->variant == DGLM_STAGE_MFMA_WS || !fp64 || (c->p.N == 4 && c->K >= WS_MIN_ELEMS)))
+    return DGLM_STAGE_MFMA_WS;
   if (c->mx_tab) return DGLM_STAGE_MFMA_MX;
   return mf ? DGLM_STAGE_MFMA : DGLM_STAGE_SIMPLE;
 }
-
-bool use_mfma(const dglm_ctx *c) { return stage_kind(c) == DGLM_STAGE_MFMA; }
 
 template <int N, int MODE>
 void launch_ws(dglm_ctx *c, const StageArgs &a) {
@@ -377,20 +391,23 @@ void launch_stage(dglm_ctx *c, const StageArgs &a) {
     launch_mx<N, MODE>(c, a);
     return;
   }
+  // the packed-column kernel; above N = 6 it is the one that goes by SIMPLE
+  if (c->p.precision == DGLM_FP64 && (kind == DGLM_STAGE_MFMA || N > 6)) {
+    c->cols.launch(MODE, c->stream, a, c->afrag_cols, c->cols_order);
+    return;
+  }
   if constexpr (N <= 6) {
     if (kind == DGLM_STAGE_MFMA) {
       if (c->p.precision == DGLM_FP32)
         launch_mfma<N, PHYS, MODE, PREC_F32>(c, a);
-      else if (c->p.precision == DGLM_BF16X3 || c->p.precision == DGLM_BF16X6)
-        launch_mfma<N, PHYS, MODE, PREC_BF>(c, a);
       else
-        launch_mfma<N, PHYS, MODE, PREC_F64>(c, a);
+        launch_mfma<N, PHYS, MODE, PREC_BF>(c, a);
       return;
     }
+    constexpr int EB = eb_simple<N, PHYS>();
+    int nblk = (c->K + EB - 1) / EB;
+    hipLaunchKernelGGL((stage_simple_kernel<N, PHYS, MODE>), dim3(nblk), dim3(256), 0, c->stream, a);
   }
-  constexpr int EB = eb_simple<N, PHYS>();
-  int nblk = (c->K + EB - 1) / EB;
-  hipLaunchKernelGGL((stage_simple_kernel<N, PHYS, MODE>), dim3(nblk), dim3(256), 0, c->stream, a);
 }
 
 typedef void (*ws_fn)(dglm_ctx *, const double *, double *, double *, int *);
@@ -477,7 +494,7 @@ void free_ctx(dglm_ctx *c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   void *ptrs[] = {c->u[0], c->u[1], c->k, c->rhs, c->vel, c->geo, c->op, c->maxv, c->partial, c->dt_hist,
                   c->conn, c->fmx, c->scal, c->afrag, c->rowsum, c->partial_idx, c->afrag_ws, c->arem_ws,
-                  c->ws_order, c->dmap, c->gbnd, c->mx_tab};
+                  c->ws_order, c->dmap, c->gbnd, c->mx_tab, c->afrag_cols, c->cols_order};
   for (void *q : ptrs)
     if (q) hipFree(q);
   free_tape(c->tape);
@@ -564,6 +581,42 @@ int scratch_on(int dev, double **out) {
 // ---------------------------------------------------------------------------
 // Context
 // ---------------------------------------------------------------------------
+// Visiting order of the batches of EB consecutive elements: by the Morton code
+// of the batch's centroid, from the corner nodes of its elements.
+static std::vector<int> batch_order(const dglm_mesh *m, int N, int Np, int EB) {
+  const int K = m->K, nb = (K + EB - 1) / EB;
+  const int corner[4] = {0, N, (N + 1) * (N + 2) / 2 - 1, Np - 1};
+  double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
+  const double *pc[3] = {m->px, m->py, m->pz};
+  std::vector<double> cen((size_t)nb * 3, 0.0);
+  for (int d = 0; d < 3; d++)
+    for (int e = 0; e < K; e++)
+      for (int q : corner) {
+        const double x = pc[d][(size_t)e * Np + q];
+        lo[d] = x < lo[d] ? x : lo[d];
+        hi[d] = x > hi[d] ? x : hi[d];
+        cen[(size_t)(e / EB) * 3 + d] += x;
+      }
+  std::vector<std::pair<unsigned long long, int>> key(nb);
+  for (int bi = 0; bi < nb; bi++) {
+    const int ne = (int)std::min((long)EB, K - (long)EB * bi);
+    unsigned long long code = 0;
+    unsigned q[3];
+    for (int d = 0; d < 3; d++) {
+      const double span = hi[d] > lo[d] ? hi[d] - lo[d] : 1.0;
+      const double t = (cen[(size_t)bi * 3 + d] / (4.0 * ne) - lo[d]) / span;
+      q[d] = (unsigned)std::min(1023.0, std::max(0.0, t * 1024.0));
+    }
+    for (int bit = 9; bit >= 0; bit--)
+      for (int d = 0; d < 3; d++) code = (code << 1) | ((q[d] >> bit) & 1u);
+    key[bi] = {code, bi};
+  }
+  std::stable_sort(key.begin(), key.end());
+  std::vector<int> order(nb);
+  for (int bi = 0; bi < nb; bi++) order[bi] = key[bi].second;
+  return order;
+}
+
 extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **out) {
   if (!p || !m || !out) return fail(DGLM_ERR_ARG, "dglm_create: null argument");
   *out = nullptr;
@@ -638,41 +691,39 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   for (int q = 0; q < NFF; q++)
     for (int i = 0; i < Np; i++) op[(size_t)(3 * Np + q) * Np + i] = -at(m->LIFT, Np, NFF, i, q);
 
-  // A-fragments of the stacked operator for the MFMA stage kernel.
-  std::vector<double> afr;
+  // Operator of the MFMA stage kernels: the streams of the packed-column kernel
+  // (FP64), or the A-fragments of the mixed-precision one.
+  const ColOps cops = cols_find(p->N, p->physics == DGLM_EULER ? PHYS_EULER : PHYS_ADV, K);
+  std::vector<double> cfr;
   std::vector<float> afr32;
   std::vector<s16x4> afrbf;
   std::vector<double> rsum;
-  if (mfma_available(p->N)) {
+  if (p->precision == DGLM_FP64) {
+    cops.fill(op.data(), cfr);
+  } else {
     const int RT = (Np + 15) / 16, KS = (KD + 3) / 4;
-    if (p->precision != DGLM_FP64) {
-      if (p->precision == DGLM_FP32) {
-        afr32.resize((size_t)RT * KS * 64);
-        arrange_a_fragments(Np, KD, RT, KS, op.data(), afr32.data());
-      } else {
-        const int KS16 = (KD + 15) / 16;
-        afrbf.resize((size_t)RT * KS16 * BF_PIECES * 64);
-        arrange_a_bf16(Np, KD, RT, KS16, op.data(), afrbf.data());
-      }
-      // affine-offset tables: [fitV (KD x 4) | fitP (KD x 4) | fitAV (Np x NBLK x 4)]
-      rsum.assign((size_t)8 * KD + (size_t)Np * NBLK * 4, 0.0);
-      std::vector<double> rx(Np), ry(Np), rz(Np);
-      for (int i = 0; i < Np; i++) {
-        rx[i] = ref.rst[i * 3];
-        ry[i] = ref.rst[i * 3 + 1];
-        rz[i] = ref.rst[i * 3 + 2];
-      }
-      if (!affine_fit_tables(Np, Nfp, ref.Fmask.data(), rx.data(), ry.data(), rz.data(), op.data(), rsum.data(),
-                             rsum.data() + 4 * KD, rsum.data() + 8 * KD))
-        return fail(DGLM_ERR_ARG, "dglm_create: singular affine-offset basis");
+    if (p->precision == DGLM_FP32) {
+      afr32.resize((size_t)RT * KS * 64);
+      arrange_a_fragments(Np, KD, RT, KS, op.data(), afr32.data());
     } else {
-      afr.resize((size_t)RT * KS * 64);
-      arrange_a_fragments(Np, KD, RT, KS, op.data(), afr.data());
+      const int KS16 = (KD + 15) / 16;
+      afrbf.resize((size_t)RT * KS16 * BF_PIECES * 64);
+      arrange_a_bf16(Np, KD, RT, KS16, op.data(), afrbf.data());
     }
+    // affine-offset tables: [fitV (KD x 4) | fitP (KD x 4) | fitAV (Np x NBLK x 4)]
+    rsum.assign((size_t)8 * KD + (size_t)Np * NBLK * 4, 0.0);
+    std::vector<double> rx(Np), ry(Np), rz(Np);
+    for (int i = 0; i < Np; i++) {
+      rx[i] = ref.rst[i * 3];
+      ry[i] = ref.rst[i * 3 + 1];
+      rz[i] = ref.rst[i * 3 + 2];
+    }
+    if (!affine_fit_tables(Np, Nfp, ref.Fmask.data(), rx.data(), ry.data(), rz.data(), op.data(), rsum.data(),
+                           rsum.data() + 4 * KD, rsum.data() + 8 * KD))
+      return fail(DGLM_ERR_ARG, "dglm_create: singular affine-offset basis");
   }
-  const size_t afrag_bytes = afr.size() * sizeof(double) + afr32.size() * sizeof(float) + afrbf.size() * sizeof(s16x4);
-  const void *afrag_src = !afr.empty() ? (const void *)afr.data()
-                                       : (!afr32.empty() ? (const void *)afr32.data() : (const void *)afrbf.data());
+  const size_t afrag_bytes = afr32.size() * sizeof(float) + afrbf.size() * sizeof(s16x4);
+  const void *afrag_src = !afr32.empty() ? (const void *)afr32.data() : (const void *)afrbf.data();
   // Operator rows for the warp-specialised FP64 Euler kernel, which also runs
   // DGLM_FP32 at the orders it is built for (N = 3, 4): there its FP64
   // contraction outruns the fused mixed-precision kernel, whose least-squares
@@ -717,41 +768,14 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
     }
   }
 
-  // Batch order of the warp-specialised kernel: 16-element batches sorted by
-  // the Morton code of their node centroid, so that the workgroups of one XCD,
-  // which walk a contiguous stretch of the order together, work on a compact
-  // region and find the neighbours' face traces in their L2.
-  std::vector<int> ws_order;
-  if ((!afr_ws.empty() || !mx_tab.empty()) && m->px && m->py && m->pz) {
-    const int nb = (K + 15) / 16;
-    const size_t KNp = (size_t)K * Np;
-    double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
-    const double *pc[3] = {m->px, m->py, m->pz};
-    std::vector<double> cen((size_t)nb * 3, 0.0);
-    for (int d = 0; d < 3; d++)
-      for (size_t i = 0; i < KNp; i++) {
-        const double x = pc[d][i];
-        lo[d] = x < lo[d] ? x : lo[d];
-        hi[d] = x > hi[d] ? x : hi[d];
-        cen[(i / Np / 16) * 3 + d] += x;
-      }
-    std::vector<std::pair<unsigned long long, int>> key(nb);
-    for (int bi = 0; bi < nb; bi++) {
-      const int ne = std::min(16, K - 16 * bi);
-      unsigned long long code = 0;
-      unsigned q[3];
-      for (int d = 0; d < 3; d++) {
-        const double span = hi[d] > lo[d] ? hi[d] - lo[d] : 1.0;
-        const double t = (cen[(size_t)bi * 3 + d] / ((double)ne * Np) - lo[d]) / span;
-        q[d] = (unsigned)std::min(1023.0, std::max(0.0, t * 1024.0));
-      }
-      for (int bit = 9; bit >= 0; bit--)
-        for (int d = 0; d < 3; d++) code = (code << 1) | ((q[d] >> bit) & 1u);
-      key[bi] = {code, bi};
-    }
-    std::stable_sort(key.begin(), key.end());
-    ws_order.resize(nb);
-    for (int bi = 0; bi < nb; bi++) ws_order[bi] = key[bi].second;
+  // Visiting orders of the batches: sorted by the Morton code of their
+  // centroid, so that the workgroups of one XCD, which walk a contiguous
+  // stretch of the order together, work on a compact region and find the
+  // neighbours' face traces in their L2.
+  std::vector<int> ws_order, cols_order;
+  if (m->px && m->py && m->pz) {
+    if (!afr_ws.empty() || !mx_tab.empty()) ws_order = batch_order(m, p->N, Np, 16);
+    if (!cfr.empty()) cols_order = batch_order(m, p->N, Np, cops.eb);
   }
 
   dglm_ctx *c = new dglm_ctx();
@@ -763,6 +787,7 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   c->KD = KD;
   c->nvar = p->physics == DGLM_EULER ? 5 : 1;
   c->dev = p->device;
+  c->cols = cops;
   c->nblk_ws = (K + wavespeed_elems(Np) - 1) / wavespeed_elems(Np);
   c->h_conn = conn;
   c->nd = (int)dface.size();
@@ -789,6 +814,8 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
       (!afr_ws.empty() && (rc = dev_alloc(&c->afrag_ws, afr_ws.size(), "A-fragments (warp-specialised)"))) ||
       (!arem_ws.empty() && (rc = dev_alloc(&c->arem_ws, arem_ws.size(), "remainder rows"))) ||
       (!ws_order.empty() && (rc = dev_alloc(&c->ws_order, ws_order.size(), "batch order"))) ||
+      (!cfr.empty() && (rc = dev_alloc(&c->afrag_cols, cfr.size(), "operator streams"))) ||
+      (!cols_order.empty() && (rc = dev_alloc(&c->cols_order, cols_order.size(), "batch order"))) ||
       (!rsum.empty() && (rc = dev_alloc(&c->rowsum, rsum.size(), "affine-offset tables"))) ||
       (!mx_tab.empty() && (rc = dev_alloc(&c->mx_tab, mx_tab.size(), "mixed-precision tables")))) {
     free_ctx(c);
@@ -822,6 +849,11 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
                  : hipSuccess,
       c->ws_order ? hipMemcpy(c->ws_order, ws_order.data(), ws_order.size() * sizeof(int), hipMemcpyHostToDevice)
                   : hipSuccess,
+      c->afrag_cols ? hipMemcpy(c->afrag_cols, cfr.data(), cfr.size() * sizeof(double), hipMemcpyHostToDevice)
+                    : hipSuccess,
+      c->cols_order ? hipMemcpy(c->cols_order, cols_order.data(), cols_order.size() * sizeof(int),
+                                hipMemcpyHostToDevice)
+                    : hipSuccess,
       c->rowsum ? hipMemcpy(c->rowsum, rsum.data(), rsum.size() * sizeof(double), hipMemcpyHostToDevice)
                 : hipSuccess,
       c->dmap ? hipMemcpy(c->dmap, dmap.data(), dmap.size() * sizeof(int), hipMemcpyHostToDevice) : hipSuccess,

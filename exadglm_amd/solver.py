@@ -165,9 +165,11 @@ class Solver:
         return dts
 
     def set_stage_kernel(self, variant):
-        """'auto', 'simple' (LDS-staged FP64), 'mfma' (one workgroup per batch,
-        operator rows in registers) or 'mfma_ws' (persistent warp-specialised
-        FP64 Euler kernel, N = 3, 4)."""
+        """'auto', 'simple' (LDS-staged FP64; the packed-column kernel above
+        N = 6), 'mfma' (FP64: packed columns; mixed precision: one workgroup
+        per batch, operator rows in registers), 'mfma_ws' (persistent
+        warp-specialised FP64 Euler kernel, N = 3, 4) or 'mfma_mx' (fused
+        mixed-precision Euler kernel)."""
         code = {"auto": A.DGLM_STAGE_AUTO, "simple": A.DGLM_STAGE_SIMPLE, "mfma": A.DGLM_STAGE_MFMA,
                 "mfma_ws": A.DGLM_STAGE_MFMA_WS, "mfma_mx": A.DGLM_STAGE_MFMA_MX}[variant]
         A.check(A.lib().dglm_set_stage_kernel(self._ctx, code))

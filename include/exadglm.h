@@ -238,15 +238,18 @@ int dglm_sync(dglm_ctx *ctx);
 int dglm_set_timing(dglm_ctx *ctx, int on);
 
 /* Stage-kernel selection (the reference picks its GPU variant by file prefix,
- * *_nopad_ / *_pad_, dglm_3d_launcher.py:176-205).  SIMPLE: LDS-staged FP64;
- * MFMA: one workgroup per 16-element batch, operator row tiles in registers
- * (N <= 6, FP64 and mixed precision); MFMA_WS: persistent warp-specialised
- * FP64 Euler kernel (producer waves stage the next batch while consumer waves
- * run the MFMA contraction; N = 3, 4, precision DGLM_FP64 or DGLM_FP32);
- * MFMA_MX: fused mixed-precision Euler kernel (DGLM_FP32, N <= 6, no
- * Dirichlet faces).  AUTO takes MFMA_WS where it exists, else MFMA_MX, else
- * MFMA, else SIMPLE (N = 7..10).  dglm_get_stage_kernel reports the kernel
- * that runs. */
+ * *_nopad_ / *_pad_, dglm_3d_launcher.py:176-205).  SIMPLE: LDS-staged FP64,
+ * scalar contraction (above N = 6 the packed-column kernel of MFMA, the only one
+ * there); MFMA (N <= 6): in FP64 the packed-column kernel (every (variable,
+ * element) pair of a batch a column of one MFMA contraction), in mixed precision
+ * one workgroup per 16-element batch, operator row tiles in registers; MFMA_WS:
+ * persistent warp-specialised FP64 Euler kernel (producer waves stage the next
+ * batch while consumer waves run the MFMA contraction; N = 3, 4, precision
+ * DGLM_FP64 or DGLM_FP32); MFMA_MX: fused mixed-precision Euler kernel
+ * (DGLM_FP32, N <= 6, no Dirichlet faces).  AUTO in FP64 takes MFMA_WS for
+ * Euler at N = 4 and K >= 20,480, else MFMA, else SIMPLE (N = 7..10); in mixed
+ * precision MFMA_WS where it exists, else MFMA_MX, else MFMA.
+ * dglm_get_stage_kernel reports the kernel that runs. */
 enum { DGLM_STAGE_AUTO = 0, DGLM_STAGE_SIMPLE = 1, DGLM_STAGE_MFMA = 2, DGLM_STAGE_MFMA_WS = 3, DGLM_STAGE_MFMA_MX = 4 };
 int dglm_set_stage_kernel(dglm_ctx *ctx, int variant);
 int dglm_get_stage_kernel(dglm_ctx *ctx, int *variant);

@@ -244,6 +244,17 @@ __device__ inline void cols_dispatch(int w, F &body) {
   }
 }
 
+// Batch of this workgroup (-1: none): workgroup i of XCD x (workgroups go to the
+// XCDs round-robin) takes entry i of the x-th eighth of the visiting order, so
+// neighbouring batches share an L2.  The grid is nbatch rounded up to a multiple
+// of 8.
+__device__ inline int xcd_batch(const int *order, int nbatch) {
+  const int xcd = blockIdx.x & 7;
+  const int slot = (int)((long)nbatch * xcd / 8) + (int)(blockIdx.x >> 3);
+  if (slot >= (int)((long)nbatch * (xcd + 1) / 8)) return -1;
+  return order ? order[slot] : slot;
+}
+
 //   MODE 0: LSRK update; MODE 1: write the RHS only.
 template <int N, int PHYS, int EB, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, const double *__restrict__ afrag,
@@ -266,13 +277,9 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   __shared__ int s_dm[EB * 4];
   __shared__ int s_fmx[16 * Nfp];
 
-  // Batch of this workgroup: workgroup i of XCD x (blocks go to the XCDs
-  // round-robin) takes entry i of the x-th eighth of the visiting order, so
-  // neighbouring batches share an L2.
-  const int xcd = blockIdx.x & 7;
-  const int slot = (int)((long)nbatch * xcd / 8) + (int)(blockIdx.x >> 3);
-  if (slot >= (int)((long)nbatch * (xcd + 1) / 8)) return;
-  const int e0 = (order ? order[slot] : slot) * EB;
+  const int batch = xcd_batch(order, nbatch);
+  if (batch < 0) return;
+  const int e0 = batch * EB;
   const int K = a.K;
   const size_t KNp = (size_t)K * Np;
   const int ne = min(EB, K - e0);
@@ -556,7 +563,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
         int v, n, o;
         place(min(i, NC * Np - VW), v, n, o);
         kr[r] = vec(0.0);
-        if (n < ne * Np) kr[r] = *reinterpret_cast<const vec *>(a.k + v * KNp + n0 + n);
+        if (a.rka != 0.0 && n < ne * Np) kr[r] = *reinterpret_cast<const vec *>(a.k + v * KNp + n0 + n);
       }
     }
     if constexpr (NA > 0) {
@@ -624,7 +631,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
           *reinterpret_cast<vec *>(a.rhs + gi) = rhs;
         } else {
           const vec kn = a.rka * kr[r] + dt * rhs;
-          *reinterpret_cast<vec *>(a.k + gi) = kn;
+          if (a.k_out) *reinterpret_cast<vec *>(a.k + gi) = kn;
           *reinterpret_cast<vec *>(a.u_out + gi) = *reinterpret_cast<const vec *>(&s_u[o]) + a.rkb * kn;
         }
       }

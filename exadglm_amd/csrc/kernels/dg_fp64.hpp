@@ -113,7 +113,10 @@ struct StageArgs {
   const double *op;   // [KD][Np]: WDr^T, WDs^T, WDt^T, -LIFT^T
   const double *maxv;
   const DevScalars *scal;
+  // The LSRK register: rka of a step's first stage is 0, so that stage need not
+  // read k, and what the last stage would write (k_out = 0) is never read.
   double rka, rkb;
+  int k_out;
   double gamma, tau_scale;
   int flux;      // 0: LM (reference), 1: Rusanov (upwind for advection)
   int bf_terms;  // split-BF16 contraction: 3 (two pieces per operand) or 6 (three pieces)
@@ -266,8 +269,8 @@ __global__ __launch_bounds__(256) void stage_simple_kernel(StageArgs a) {
     if (MODE == 1) {
       a.rhs[gi] = acc;
     } else {
-      const double kn = a.rka * a.k[gi] + dt * acc;
-      a.k[gi] = kn;
+      const double kn = (a.rka != 0.0 ? a.rka * a.k[gi] : 0.0) + dt * acc;
+      if (a.k_out) a.k[gi] = kn;
       a.u_out[gi] = s_u[v][r] + a.rkb * kn;
     }
   }

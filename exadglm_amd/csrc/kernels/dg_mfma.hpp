@@ -536,8 +536,8 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
             if (MODE == 1) {
               a.rhs[gi] = rhs;
             } else {
-              const double kn = a.rka * a.k[gi] + dt * rhs;
-              a.k[gi] = kn;
+              const double kn = (a.rka != 0.0 ? a.rka * a.k[gi] : 0.0) + dt * rhs;
+              if (a.k_out) a.k[gi] = kn;
               a.u_out[gi] = s_u[v][e * Np + i] + a.rkb * kn;
             }
           }

@@ -575,7 +575,7 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
       const size_t g0 = v * KNp + (size_t)(e0 + ec) * Np + i0;
       const bool full = i0 + 3 < Np;
       double kold[4] = {0.0, 0.0, 0.0, 0.0};
-      if (MODE == 0 && ec < ne) {
+      if (MODE == 0 && a.rka != 0.0 && ec < ne) {
         if (full) {
           const f64x2u k01 = *reinterpret_cast<const f64x2u *>(a.k + g0);
           const f64x2u k23 = *reinterpret_cast<const f64x2u *>(a.k + g0 + 2);
@@ -618,8 +618,10 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
         }
         double *d1 = MODE == 1 ? a.rhs : a.k;
         if (full) {
-          *reinterpret_cast<f64x2u *>(d1 + g0) = f64x2u{o1[0], o1[1]};
-          *reinterpret_cast<f64x2u *>(d1 + g0 + 2) = f64x2u{o1[2], o1[3]};
+          if (MODE == 1 || a.k_out) {
+            *reinterpret_cast<f64x2u *>(d1 + g0) = f64x2u{o1[0], o1[1]};
+            *reinterpret_cast<f64x2u *>(d1 + g0 + 2) = f64x2u{o1[2], o1[3]};
+          }
           if (MODE == 0) {
             *reinterpret_cast<f64x2u *>(a.u_out + g0) = f64x2u{o2[0], o2[1]};
             *reinterpret_cast<f64x2u *>(a.u_out + g0 + 2) = f64x2u{o2[2], o2[3]};

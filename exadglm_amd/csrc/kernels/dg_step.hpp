@@ -1,5 +1,5 @@
 // Per-step reductions that are plain (non-template) kernels: the device-side
-// dt and the conserved integrals.  Included by solver.hip only, so each is
+// dt, its adjoint and the conserved integrals.  Included by solver.hip only, so each is
 // defined in one translation unit.
 //   calc_dt  dim3/src/cpp/euler_dglm.cpp:53-69, euler_time.cpp:49-57
 #pragma once
@@ -89,6 +89,32 @@ __global__ __launch_bounds__(256) void integrals_kernel(int K, int Np, int nvar,
     }
     if (threadIdx.x == 0) partial[(size_t)blockIdx.x * nvar + v] = red[0];
     __syncthreads();
+  }
+}
+
+// dtbar of the step = sum of the block partials + tbar (adjoint of the time
+// after the step).  If the step was clipped to end at tmax, dt = tmax - t
+// does not depend on the wave speed and its adjoint flows into t instead.
+// One block; scal[0] = tbar (in/out), scal[1] = dtbar seen by lambda (out).
+__global__ __launch_bounds__(256) void adjoint_dt_reduce(const double *__restrict__ dtpart, int n,
+                                                         const int *__restrict__ clipped, int step, double *scal) {
+  __shared__ double red[256];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) s += dtpart[i];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const double dtbar = red[0] + scal[0];
+    if (clipped[step]) {
+      scal[0] -= dtbar;
+      scal[1] = 0.0;
+    } else {
+      scal[1] = dtbar;
+    }
   }
 }
 

@@ -460,6 +460,7 @@ __device__ inline void ws_consume(const StageArgs &a, WsSlot<N> *sl, const doubl
   }
   const double *afs = s_afs + (size_t)t * KSS * 64 + lane;
   const double *fsv = fs + v * NFF4 * S::FS;
+  const bool kin = a.rka != 0.0;
 
   for (int it = 0; b < hi; b += gsz, it++) {
     const WsSlot<N> &s = sl[it & 1];
@@ -471,11 +472,11 @@ __device__ inline void ws_consume(const StageArgs &a, WsSlot<N> *sl, const doubl
     double kp[4], kpr[RR > 0 ? RR : 1];
     if (MODE == 0) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) kp[r] = live ? a.k[gbase + 16 * t + 4 * r + kk] : 0.0;
+      for (int r = 0; r < 4; r++) kp[r] = kin && live ? a.k[gbase + 16 * t + 4 * r + kk] : 0.0;
 #pragma unroll
       for (int x = 0; x < RR; x++) {
         const int rr = kk + 4 * x;
-        kpr[x] = (live && rr < REM) ? a.k[gbase + 16 * RTF + RLO + rr] : 0.0;
+        kpr[x] = (kin && live && rr < REM) ? a.k[gbase + 16 * RTF + RLO + rr] : 0.0;
       }
     }
     // The remainder-row operator values are the same every batch; an opaque
@@ -561,7 +562,7 @@ __device__ inline void ws_consume(const StageArgs &a, WsSlot<N> *sl, const doubl
           a.rhs[gi] = rhs;
         } else {
           const double kn = a.rka * kp[r] + dt * rhs;
-          a.k[gi] = kn;
+          if (a.k_out) a.k[gi] = kn;
           a.u_out[gi] = s.u[v][e * Np + i] + a.rkb * kn;
         }
       }
@@ -587,7 +588,7 @@ __device__ inline void ws_consume(const StageArgs &a, WsSlot<N> *sl, const doubl
             a.rhs[gi] = rhs;
           } else {
             const double kn = a.rka * kpr[x] + dt * rhs;
-            a.k[gi] = kn;
+            if (a.k_out) a.k[gi] = kn;
             a.u_out[gi] = s.u[v][e * Np + i] + a.rkb * kn;
           }
         }

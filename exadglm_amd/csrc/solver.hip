@@ -29,8 +29,8 @@
 #include "kernels/dg_mfma.hpp"
 #include "kernels/dg_ws.hpp"
 #include "kernels/dg_mx.hpp"
+#include "kernels/adjoint_ops.h"
 #include "kernels/dg_adjoint.hpp"
-#include "kernels/dg_adjoint_mfma.hpp"
 
 namespace dglm {
 // ws_dirichlet.hip: the warp-specialised stage kernel on meshes with Dirichlet
@@ -105,6 +105,7 @@ struct dglm_ctx {
   bool adj_exact = true;          // include the tau(u) and dt(u) sensitivities (Euler)
   int adj_keep_max = -1;          // segments kept whole on the tape (-1: as many as half the free HBM holds)
   std::vector<int> h_conn;  // host copy (tau pairing for the rhs outputs)
+  std::vector<float> h_centroid;  // element centroids (visiting orders; empty: mesh order)
   // Dirichlet faces (EtoB == 1): slot map [K*4] (-1: none), prescribed states
   // [nvar][nd][Nfp] and the faces of the slots in ascending order.
   int nd = 0;
@@ -459,6 +460,7 @@ StageArgs stage_args(dglm_ctx *c, int s) {
   a.scal = c->scal;
   a.rka = s >= 0 ? RKA[s] : 0.0;
   a.rkb = s >= 0 ? RKB[s] : 0.0;
+  a.k_out = s != 4;
   a.gamma = c->p.gamma;
   a.tau_scale = c->p.tau_scale;
   a.flux = c->p.flux == DGLM_FLUX_RUSANOV ? 1 : 0;
@@ -581,30 +583,48 @@ int scratch_on(int dev, double **out) {
 // ---------------------------------------------------------------------------
 // Context
 // ---------------------------------------------------------------------------
-// Visiting order of the batches of EB consecutive elements: by the Morton code
-// of the batch's centroid, from the corner nodes of its elements.
-static std::vector<int> batch_order(const dglm_mesh *m, int N, int Np, int EB) {
-  const int K = m->K, nb = (K + EB - 1) / EB;
-  const int corner[4] = {0, N, (N + 1) * (N + 2) / 2 - 1, Np - 1};
-  double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
+// Element centroids (of their corner nodes), scaled to the mesh's bounding box;
+// empty without node coordinates.
+static std::vector<float> element_centroids(const dglm_mesh *m, int N, int Np) {
+  std::vector<float> cen;
+  if (!m->px || !m->py || !m->pz) return cen;
+  const int K = m->K, corner[4] = {0, N, (N + 1) * (N + 2) / 2 - 1, Np - 1};
+  cen.resize((size_t)K * 3);
   const double *pc[3] = {m->px, m->py, m->pz};
-  std::vector<double> cen((size_t)nb * 3, 0.0);
-  for (int d = 0; d < 3; d++)
+  for (int d = 0; d < 3; d++) {
+    double lo = HUGE_VAL, hi = -HUGE_VAL;
     for (int e = 0; e < K; e++)
       for (int q : corner) {
         const double x = pc[d][(size_t)e * Np + q];
-        lo[d] = x < lo[d] ? x : lo[d];
-        hi[d] = x > hi[d] ? x : hi[d];
-        cen[(size_t)(e / EB) * 3 + d] += x;
+        lo = x < lo ? x : lo;
+        hi = x > hi ? x : hi;
       }
+    const double scale = hi > lo ? 0.25 / (hi - lo) : 0.0;
+    for (int e = 0; e < K; e++) {
+      double sum = 0.0;
+      for (int q : corner) sum += pc[d][(size_t)e * Np + q] - lo;
+      cen[(size_t)e * 3 + d] = (float)(sum * scale);
+    }
+  }
+  return cen;
+}
+
+// Visiting order of the batches of EB consecutive elements: by the Morton code
+// of the batch's centroid, so that the workgroups of one XCD, which walk a
+// contiguous stretch of the order together, work on a compact region and find
+// the neighbours' face traces in their L2.
+static std::vector<int> batch_order(const std::vector<float> &elem, int EB) {
+  const int K = (int)(elem.size() / 3), nb = (K + EB - 1) / EB;
+  std::vector<double> cen((size_t)nb * 3, 0.0);
+  for (int e = 0; e < K; e++)
+    for (int d = 0; d < 3; d++) cen[(size_t)(e / EB) * 3 + d] += elem[(size_t)e * 3 + d];
   std::vector<std::pair<unsigned long long, int>> key(nb);
   for (int bi = 0; bi < nb; bi++) {
     const int ne = (int)std::min((long)EB, K - (long)EB * bi);
     unsigned long long code = 0;
     unsigned q[3];
     for (int d = 0; d < 3; d++) {
-      const double span = hi[d] > lo[d] ? hi[d] - lo[d] : 1.0;
-      const double t = (cen[(size_t)bi * 3 + d] / (4.0 * ne) - lo[d]) / span;
+      const double t = cen[(size_t)bi * 3 + d] / ne;
       q[d] = (unsigned)std::min(1023.0, std::max(0.0, t * 1024.0));
     }
     for (int bit = 9; bit >= 0; bit--)
@@ -768,14 +788,12 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
     }
   }
 
-  // Visiting orders of the batches: sorted by the Morton code of their
-  // centroid, so that the workgroups of one XCD, which walk a contiguous
-  // stretch of the order together, work on a compact region and find the
-  // neighbours' face traces in their L2.
+  // Visiting orders of the batches.
+  std::vector<float> centroid = element_centroids(m, p->N, Np);
   std::vector<int> ws_order, cols_order;
-  if (m->px && m->py && m->pz) {
-    if (!afr_ws.empty() || !mx_tab.empty()) ws_order = batch_order(m, p->N, Np, 16);
-    if (!cfr.empty()) cols_order = batch_order(m, p->N, Np, cops.eb);
+  if (!centroid.empty()) {
+    if (!afr_ws.empty() || !mx_tab.empty()) ws_order = batch_order(centroid, 16);
+    if (!cfr.empty()) cols_order = batch_order(centroid, cops.eb);
   }
 
   dglm_ctx *c = new dglm_ctx();
@@ -788,6 +806,7 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   c->nvar = p->physics == DGLM_EULER ? 5 : 1;
   c->dev = p->device;
   c->cols = cops;
+  c->h_centroid.swap(centroid);
   c->nblk_ws = (K + wavespeed_elems(Np) - 1) / wavespeed_elems(Np);
   c->h_conn = conn;
   c->nd = (int)dface.size();
@@ -861,7 +880,6 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
       hipMemcpy(c->scal, &s0, sizeof(s0), hipMemcpyHostToDevice),
       hipMemset(c->u[0], 0, nst * sizeof(double)),
       hipMemset(c->u[1], 0, nst * sizeof(double)),
-      hipMemset(c->k, 0, nst * sizeof(double)),
   };
   for (hipError_t e : errs)
     if (e != hipSuccess) {
@@ -929,7 +947,7 @@ static int set_state_impl(dglm_ctx *c, const double *u, hipMemcpyKind kind) {
   const size_t n = (size_t)c->nvar * c->K * c->Np;
   c->cur = 0;
   HIP_TRY(hipMemcpyAsync(c->u[0], u, n * sizeof(double), kind, c->stream));
-  HIP_TRY(hipMemsetAsync(c->k, 0, n * sizeof(double), c->stream));
+  // (the LSRK register needs no clearing: a step's first stage does not read it)
   HIP_TRY(hipStreamSynchronize(c->stream));
   return DGLM_OK;
 }
@@ -1300,15 +1318,6 @@ typedef void (*adj_fn)(dglm_ctx *, const AdjArgs &);
 typedef void (*lam_fn)(dglm_ctx *, const double *, const double *, int);
 
 template <int N, int PHYS>
-void launch_adj_a(dglm_ctx *c, const AdjArgs &a) {
-  constexpr int EB = eb_adjoint<N, PHYS>();
-  hipLaunchKernelGGL((adjoint_pass_a<N, PHYS>), dim3((c->K + EB - 1) / EB), dim3(256), 0, c->stream, a);
-}
-
-template <int N>
-void launch_adj_a_mfma(dglm_ctx *c, const AdjArgs &a);
-
-template <int N, int PHYS>
 void launch_adj_b(dglm_ctx *c, const AdjArgs &a) {
   const int n = c->K * Ord<N>::Np;
   hipLaunchKernelGGL((adjoint_pass_b<N, PHYS>), dim3((n + 255) / 256), dim3(256), 0, c->stream, a);
@@ -1317,52 +1326,13 @@ void launch_adj_b(dglm_ctx *c, const AdjArgs &a) {
 template <int N>
 void launch_lam(dglm_ctx *c, const double *u, const double *lam, int step);
 
-template <int N, int PHYS>
-int adj_blocks() {
-  constexpr int EB = eb_adjoint<N, PHYS>();
-  return EB;
-}
-
-// The MFMA pass A (FP64 Euler, N <= 4) where it fits a workgroup.
 template <int PHYS>
-bool pick_adj_mfma(int N, adj_fn &A, int &eb) {
-  if (PHYS != PHYS_EULER) return false;
-  switch (N) {
-#define DGLM_MCASE(n)                          \
-  case n:                                      \
-    if (!adj_mfma_available<n>()) return false; \
-    A = launch_adj_a_mfma<n>;                  \
-    eb = AdjShape<n>::EB;                      \
-    return true;
-    DGLM_MCASE(1)
-    DGLM_MCASE(2)
-    DGLM_MCASE(3)
-    DGLM_MCASE(4)
-#undef DGLM_MCASE
-    default:
-      return false;
-  }
-}
-
-template <int PHYS>
-bool pick_adj_impl(int N, adj_fn &A, adj_fn &B, lam_fn &Lf, int &eb);
-
-template <int PHYS>
-bool pick_adj(int N, adj_fn &A, adj_fn &B, lam_fn &Lf, int &eb) {
-  if (!pick_adj_impl<PHYS>(N, A, B, Lf, eb)) return false;
-  pick_adj_mfma<PHYS>(N, A, eb);
-  return true;
-}
-
-template <int PHYS>
-bool pick_adj_impl(int N, adj_fn &A, adj_fn &B, lam_fn &Lf, int &eb) {
+bool pick_adj(int N, adj_fn &B, lam_fn &Lf) {
   switch (N) {
 #define DGLM_ACASE(n)                      \
   case n:                                  \
-    A = launch_adj_a<n, PHYS>;             \
     B = launch_adj_b<n, PHYS>;             \
     Lf = launch_lam<n>;                    \
-    eb = adj_blocks<n, PHYS>();            \
     return true;
     DGLM_ACASE(1)
     DGLM_ACASE(2)
@@ -1380,6 +1350,10 @@ bool pick_adj_impl(int N, adj_fn &A, adj_fn &B, lam_fn &Lf, int &eb) {
   }
 }
 
+bool adj_dispatch(const dglm_ctx *c, adj_fn &B, lam_fn &Lf) {
+  return c->p.physics == DGLM_EULER ? pick_adj<PHYS_EULER>(c->p.N, B, Lf) : pick_adj<PHYS_ADV>(c->p.N, B, Lf);
+}
+
 StageArgs make_stage_args(dglm_ctx *c, const double *u_in, double *u_out, double *k, const double *maxv,
                           const DevScalars *scal, int s) {
   StageArgs a = stage_args(c, s);
@@ -1394,36 +1368,28 @@ StageArgs make_stage_args(dglm_ctx *c, const double *u_in, double *u_out, double
 }  // namespace
 
 struct dglm_adj_tape {
-  int nsteps = 0, every = 0, nck = 0, eb = 1, nblk_a = 0;
-  double *afragT = nullptr;  // A^T fragments of the MFMA pass A (null: scalar pass A)
+  int nsteps = 0, every = 0, nck = 0, nblk_a = 0;
+  AdjOps ops;                // pass A of this order and physics
+  double *afragT = nullptr;  // its operator streams
+  int *order = nullptr;      // its batch visiting order (null: mesh order)
   double *ckpt = nullptr, *ck_t = nullptr, *dt = nullptr, *seg = nullptr, *lam = nullptr, *kscr = nullptr;
   int *fstar = nullptr, *clip = nullptr, *ck_step = nullptr;
   DevScalars *scal2 = nullptr;
   double *ubar = nullptr, *kbar = nullptr, *gsur = nullptr, *taubar = nullptr, *dtpart = nullptr, *tsc = nullptr;
-  // second face-term buffer of the MFMA pass A, which takes over the pass B
-  // of stages 4..1 (each pass A reads the terms of the one before it while
-  // writing its own)
+  // second face-term buffer: each pass A reads the terms of the one before it
+  // while writing its own
   double *gsur2 = nullptr;
   double *rbar = nullptr;
-  int *slots = nullptr, *fpos = nullptr;
+  int *slots = nullptr, *pslot = nullptr;
   // The last nkeep segments kept whole: their stage states [5*every + 1][nst]
   // and wave speeds [every][K*4] per segment, written by the recording
   // forward itself, so the reverse sweep does not recompute them.
   double *keep = nullptr, *keep_lam = nullptr;
   int nkeep = 0;
-  size_t bytes = 0, keep_bytes = 0;
+  size_t bytes = 0, base_bytes = 0, keep_bytes = 0;  // the whole tape, without a recording, its kept segments
 };
 
 namespace {
-
-template <int N>
-void launch_adj_a_mfma(dglm_ctx *c, const AdjArgs &a) {
-  if constexpr (adj_mfma_available<N>()) {
-    using S = AdjShape<N>;
-    hipLaunchKernelGGL((adjoint_pass_a_mfma<N>), dim3((c->K + S::EB - 1) / S::EB), dim3(S::NT), 0, c->stream, a,
-                       c->tape->afragT);
-  }
-}
 
 template <int N>
 void launch_lam(dglm_ctx *c, const double *u, const double *lam, int step) {
@@ -1437,8 +1403,8 @@ void launch_lam(dglm_ctx *c, const double *u, const double *lam, int step) {
 void free_tape(dglm_adj_tape *T) {
   if (!T) return;
   void *ptrs[] = {T->keep, T->keep_lam, T->ckpt, T->ck_t, T->dt, T->seg, T->lam, T->kscr, T->fstar, T->clip, T->ck_step, T->scal2,
-                  T->ubar, T->kbar, T->gsur, T->gsur2, T->taubar, T->dtpart, T->tsc, T->rbar, T->slots, T->fpos,
-                  T->afragT};
+                  T->ubar, T->kbar, T->gsur, T->gsur2, T->taubar, T->dtpart, T->tsc, T->rbar, T->slots, T->pslot,
+                  T->afragT, T->order};
   for (void *q : ptrs)
     if (q) hipFree(q);
   delete T;
@@ -1449,20 +1415,16 @@ int ensure_adjoint_buffers(dglm_ctx *c) {
   if (!c->tape) c->tape = new dglm_adj_tape();
   dglm_adj_tape *T = c->tape;
   if (T->ubar) return DGLM_OK;
-  adj_fn A, B;
-  lam_fn L;
-  int eb = 1;
-  bool ok = c->p.physics == DGLM_EULER ? pick_adj<PHYS_EULER>(c->p.N, A, B, L, eb)
-                                       : pick_adj<PHYS_ADV>(c->p.N, A, B, L, eb);
-  if (!ok) return fail(DGLM_ERR_UNSUPPORTED, "adjoint: order not built");
-  T->eb = eb;
-  T->nblk_a = (c->K + eb - 1) / eb;
-  const size_t nst = (size_t)c->nvar * c->K * c->Np;
-  // face-node slots of each volume node, and node positions in each face mask
+  T->ops = c->p.physics == DGLM_EULER ? adjoint_euler(c->p.N) : adjoint_advection(c->p.N);
+  if (!T->ops.eb) return fail(DGLM_ERR_UNSUPPORTED, "adjoint: order not built");
+  T->nblk_a = (c->K + T->ops.eb - 1) / T->ops.eb;
+  const size_t nst = (size_t)c->nvar * c->K * c->Np, ng = (size_t)c->nvar * c->K * c->NFF;
+  // face-node slots of each volume node, and the neighbour's slot of each entry
+  // (face, code, j) of the face-node table
   RefOps ref;
   reference_operators(c->p.N, ref);
   const int Np = c->Np, Nfp = c->Nfp;
-  std::vector<int> slots((size_t)Np * 3, -1), fpos((size_t)4 * Np, -1);
+  std::vector<int> slots((size_t)Np * 3, -1), pslot((size_t)16 * Nfp, 0);
   for (int m = 0; m < 4 * Nfp; m++) {
     const int node = ref.Fmask[m];
     for (int q = 0; q < 3; q++)
@@ -1470,44 +1432,35 @@ int ensure_adjoint_buffers(dglm_ctx *c) {
         slots[node * 3 + q] = m;
         break;
       }
-    fpos[(m / Nfp) * Np + node] = m % Nfp;
   }
+  for (int f = 0; f < 4; f++)
+    for (int cde = 0; cde < 4; cde++)
+      for (int j = 0; j < Nfp; j++) {
+        const int node = cde < 3 ? ref.FmaskP[(f * 3 + cde) * Nfp + j] : ref.Fmask[f * Nfp + j];
+        for (int jp = 0; jp < Nfp; jp++)
+          if (ref.Fmask[f * Nfp + jp] == node) pslot[(f * 4 + cde) * Nfp + j] = f * Nfp + jp;
+      }
+  std::vector<double> opT((size_t)c->KD * Np), frag;
+  HIP_TRY(hipMemcpy(opT.data(), c->op, opT.size() * sizeof(double), hipMemcpyDeviceToHost));
+  T->ops.fill(opT.data(), frag);
+  std::vector<int> order;
+  if (!c->h_centroid.empty()) order = batch_order(c->h_centroid, T->ops.eb);
   int rc;
-  if ((rc = dev_alloc(&T->ubar, nst, "ubar")) || (rc = dev_alloc(&T->kbar, nst, "kbar")) ||
-      (rc = dev_alloc(&T->gsur, (size_t)c->nvar * c->K * c->NFF, "face adjoint")) ||
-      (rc = dev_alloc(&T->taubar, (size_t)c->K * 4, "taubar")) ||
-      (rc = dev_alloc(&T->dtpart, (size_t)T->nblk_a, "dt partials")) || (rc = dev_alloc(&T->tsc, 4, "t scalars")) ||
-      (rc = dev_alloc(&T->slots, slots.size(), "node slots")) || (rc = dev_alloc(&T->fpos, fpos.size(), "fpos")))
+  // (a call after a failed one allocates what that one could not; ubar last)
+  auto need = [](auto **p, size_t n, const char *what) { return *p ? DGLM_OK : dev_alloc(p, n, what); };
+  if ((rc = need(&T->kbar, nst, "kbar")) || (rc = need(&T->gsur, ng, "face adjoint")) ||
+      (rc = need(&T->gsur2, ng, "face adjoint (second)")) || (rc = need(&T->taubar, (size_t)c->K * 4, "taubar")) ||
+      (rc = need(&T->dtpart, (size_t)T->nblk_a, "dt partials")) || (rc = need(&T->tsc, 4, "t scalars")) ||
+      (rc = need(&T->slots, slots.size(), "node slots")) || (rc = need(&T->pslot, pslot.size(), "partner slots")) ||
+      (!order.empty() && (rc = need(&T->order, order.size(), "batch order"))) ||
+      (rc = need(&T->afragT, frag.size(), "A^T operator streams")) || (rc = need(&T->ubar, nst, "ubar")))
     return rc;
   HIP_TRY(hipMemcpy(T->slots, slots.data(), slots.size() * sizeof(int), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(T->fpos, fpos.data(), fpos.size() * sizeof(int), hipMemcpyHostToDevice));
-  T->bytes += (2 * nst + (size_t)c->nvar * c->K * c->NFF + (size_t)c->K * 4 + T->nblk_a) * sizeof(double);
-  // A^T fragments for the MFMA pass A
-  adj_fn Am;
-  int ebm = 0;
-  if (c->p.physics == DGLM_EULER && pick_adj_mfma<PHYS_EULER>(c->p.N, Am, ebm)) {
-    std::vector<double> opT((size_t)c->KD * Np), frag;
-    HIP_TRY(hipMemcpy(opT.data(), c->op, opT.size() * sizeof(double), hipMemcpyDeviceToHost));
-    switch (c->p.N) {
-#define DGLM_FCASE(n)                                                            \
-  case n:                                                                        \
-    frag.resize((size_t)AdjShape<n>::KT * AdjShape<n>::KSA * 64);               \
-    adj_arrange<n>(opT.data(), frag.data());                                     \
-    break;
-      DGLM_FCASE(1)
-      DGLM_FCASE(2)
-      DGLM_FCASE(3)
-      DGLM_FCASE(4)
-#undef DGLM_FCASE
-      default:
-        break;
-    }
-    if ((rc = dev_alloc(&T->afragT, frag.size(), "A^T fragments"))) return rc;
-    HIP_TRY(hipMemcpy(T->afragT, frag.data(), frag.size() * sizeof(double), hipMemcpyHostToDevice));
-    const size_t ng = (size_t)c->nvar * c->K * c->NFF;
-    if ((rc = dev_alloc(&T->gsur2, ng, "face adjoint (second)"))) return rc;
-    T->bytes += ng * sizeof(double);
-  }
+  HIP_TRY(hipMemcpy(T->pslot, pslot.data(), pslot.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (!order.empty()) HIP_TRY(hipMemcpy(T->order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(T->afragT, frag.data(), frag.size() * sizeof(double), hipMemcpyHostToDevice));
+  T->base_bytes = (2 * nst + 2 * ng + (size_t)c->K * 4 + T->nblk_a) * sizeof(double);
+  T->bytes = T->base_bytes;
   return DGLM_OK;
 }
 
@@ -1524,8 +1477,8 @@ AdjArgs adj_args(dglm_ctx *c) {
   a.conn = c->conn;
   a.fmx = c->fmx;
   a.node_slots = T->slots;
-  a.fpos = T->fpos;
-  a.op = c->op;
+  a.pslot = T->pslot;
+  a.order = T->order;
   a.gamma = c->p.gamma;
   a.tau_scale = c->p.tau_scale;
   return a;
@@ -1545,12 +1498,10 @@ extern "C" int dglm_adjoint_rhs(dglm_ctx *c, const double *u, const double *rbar
   if (!T->rbar && (rc = dev_alloc(&T->rbar, nst, "rbar"))) return rc;
   ws_fn ws;
   st_fn st0, st1;
-  adj_fn A, B;
+  adj_fn B;
   lam_fn L;
-  int eb;
-  if (!dispatch(c, ws, st0, st1)) return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_rhs: order not built");
-  if (c->p.physics == DGLM_EULER) pick_adj<PHYS_EULER>(c->p.N, A, B, L, eb);
-  else pick_adj<PHYS_ADV>(c->p.N, A, B, L, eb);
+  if (!dispatch(c, ws, st0, st1) || !adj_dispatch(c, B, L))
+    return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_rhs: order not built");
   HIP_TRY(hipMemcpyAsync(c->u[c->cur], u, nst * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipMemcpyAsync(T->rbar, rbar, nst * sizeof(double), hipMemcpyHostToDevice, c->stream));
   ws(c, c->u[c->cur], c->maxv, c->partial, c->partial_idx);  // tau at u
@@ -1559,7 +1510,7 @@ extern "C" int dglm_adjoint_rhs(dglm_ctx *c, const double *u, const double *rbar
   a.u = c->u[c->cur];
   a.rbar = T->rbar;
   a.maxv = c->maxv;
-  A(c, a);
+  T->ops.launch(c->stream, a, T->afragT);
   B(c, a);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(ubar, T->ubar, nst * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1582,6 +1533,24 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
   if (!dispatch(c, ws, st0, st1)) return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_record: order not built");
   const size_t nst = (size_t)c->nvar * c->K * c->Np;
   const int nck = (nsteps + every - 1) / every;
+  const double cfl_fac = c->p.cfl / (2 * c->p.N + 1);
+  if (c->p.physics == DGLM_ADVECTION) {
+    // Linear: the reverse sweep needs dt of every step and the (constant) wave
+    // speeds, no states.
+    if (T->nsteps != nsteps) {
+      T->nsteps = 0;
+      if (T->dt) HIP_TRY(hipFree(T->dt));
+      T->dt = nullptr;
+      if (!T->lam && (rc = dev_alloc(&T->lam, (size_t)c->K * 4, "wave speeds"))) return rc;
+      if ((rc = dev_alloc(&T->dt, (size_t)nsteps, "dt"))) return rc;
+      T->nsteps = nsteps;
+      T->bytes = T->base_bytes + ((size_t)c->K * 4 + nsteps) * sizeof(double);
+    }
+    for (int n = 0; n < nsteps; n++) enqueue_step(c, ws, st0, T->dt, n, c->partial, c->partial_idx, false);
+    HIP_TRY(hipMemcpyAsync(T->lam, c->maxv, (size_t)c->K * 4 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    HIP_TRY(hipGetLastError());
+    return DGLM_OK;
+  }
   // (re)allocate the recording buffers when the shape changes
   if (T->nsteps != nsteps || T->every != every) {
     // The tape is empty until every buffer of the new shape exists: a failed
@@ -1609,9 +1578,7 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
     T->nsteps = nsteps;
     T->every = every;
     T->nck = nck;
-    T->bytes = (2 * nst + (size_t)c->nvar * c->K * c->NFF * (T->gsur2 ? 2 : 1) + (size_t)c->K * 4 + T->nblk_a) *
-                   sizeof(double) +
-               (nst * (nck + 5 * (size_t)every + 2) + (size_t)c->K * 4 * every) * sizeof(double);
+    T->bytes = T->base_bytes + (nst * (nck + 5 * (size_t)every + 2) + (size_t)c->K * 4 * every) * sizeof(double);
   }
   // Segments kept whole: HBM bought back from the recompute.  The count is the
   // caller's cap (dglm_adjoint_set_keep) or, by default, what half of the free
@@ -1649,7 +1616,6 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
     }
   }
   const int q0 = nck - T->nkeep;  // first kept segment
-  const double cfl_fac = c->p.cfl / (2 * c->p.N + 1);
   for (int n = 0; n < nsteps; n++) {
     const int q = n / every;
     if (n % every == 0) {
@@ -1703,25 +1669,26 @@ extern "C" int dglm_adjoint_backward(dglm_ctx *c, const double *ubar_T, double *
   HIP_TRY(hipSetDevice(c->dev));
   ws_fn ws;
   st_fn st0, st1;
-  adj_fn A, B;
+  adj_fn B;
   lam_fn L;
-  int eb;
-  if (!dispatch(c, ws, st0, st1)) return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_backward: order not built");
-  if (c->p.physics == DGLM_EULER) pick_adj<PHYS_EULER>(c->p.N, A, B, L, eb);
-  else pick_adj<PHYS_ADV>(c->p.N, A, B, L, eb);
+  if (!dispatch(c, ws, st0, st1) || !adj_dispatch(c, B, L))
+    return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_backward: order not built");
   const size_t nst = (size_t)c->nvar * c->K * c->Np;
-  const bool exact = c->adj_exact && c->p.physics == DGLM_EULER;
+  const bool linear = c->p.physics == DGLM_ADVECTION;
+  const bool exact = c->adj_exact && !linear;
   const double cfl_fac = c->p.cfl / (2 * c->p.N + 1);
   const hipMemcpyKind kin = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   HIP_TRY(hipMemcpyAsync(T->ubar, ubar_T, nst * sizeof(double), kin, c->stream));
-  HIP_TRY(hipMemsetAsync(T->kbar, 0, nst * sizeof(double), c->stream));
-  HIP_TRY(hipMemsetAsync(T->kscr, 0, nst * sizeof(double), c->stream));
   HIP_TRY(hipMemsetAsync(T->tsc, 0, 4 * sizeof(double), c->stream));
-  const int q0 = T->nck - std::max(T->nkeep, 0);  // first segment kept whole by the recording
-  for (int q = T->nck - 1; q >= 0; q--) {
-    const int n0 = q * T->every, n1 = std::min(n0 + T->every, T->nsteps);
+  const double *pend = nullptr;  // partner terms of the last pass A, not yet added
+  const int every = linear ? T->nsteps : T->every, nck = linear ? 1 : T->nck;
+  const int q0 = nck - std::max(T->nkeep, 0);  // first segment kept whole by the recording
+  for (int q = nck - 1; q >= 0; q--) {
+    const int n0 = q * every, n1 = std::min(n0 + every, T->nsteps);
     double *seg = T->seg, *segl = T->lam;
-    if (q >= q0) {
+    if (linear) {
+      // no states to recompute
+    } else if (q >= q0) {
       seg = T->keep + nst * (5 * (size_t)T->every + 1) * (q - q0);
       segl = T->keep_lam + (size_t)c->K * 4 * T->every * (q - q0);
     } else {
@@ -1742,41 +1709,38 @@ extern "C" int dglm_adjoint_backward(dglm_ctx *c, const double *ubar_T, double *
     }
     // reverse sweep over the segment
     for (int n = n1 - 1; n >= n0; n--) {
-      double *base = seg + nst * 5 * (size_t)(n - n0);
-      const double *lam = segl + (size_t)c->K * 4 * (n - n0);
-      HIP_TRY(hipMemsetAsync(T->taubar, 0, (size_t)c->K * 4 * sizeof(double), c->stream));
-      HIP_TRY(hipMemsetAsync(T->dtpart, 0, (size_t)T->nblk_a * sizeof(double), c->stream));
-      for (int s = 4; s >= 0; s--) {
+      double *base = linear ? nullptr : seg + nst * 5 * (size_t)(n - n0);
+      const double *lam = linear ? segl : segl + (size_t)c->K * 4 * (n - n0);
+      for (int st = 4; st >= 0; st--) {
         AdjArgs a = adj_args(c);
         a.mode = 0;
-        if (T->gsur2) {
-          // the MFMA pass A adds the partner terms of the stage before it
-          // (written to the other buffer); only stage 0's go through pass B,
-          // ahead of the wave-speed adjoint
-          a.gsur = (s & 1) ? T->gsur2 : T->gsur;
-          a.gsur_in = s < 4 ? ((s & 1) ? T->gsur : T->gsur2) : nullptr;
-        }
-        a.u = base + nst * s;
+        a.first = st == 4;
+        // each pass A adds the partner terms that the one before it wrote to
+        // the other buffer
+        a.gsur = pend == T->gsur ? T->gsur2 : T->gsur;
+        a.gsur_in = pend;
+        a.u = linear ? nullptr : base + nst * st;
         a.maxv = lam;
         a.dtp = T->dt + n;
-        a.a = RKA[s];
-        a.b = RKB[s];
-        if (exact) {
-          a.u_next = base + nst * (s + 1);
-          a.u_prev = s > 0 ? base + nst * (s - 1) : nullptr;
-          a.a_prev = s > 0 ? RKA[s - 1] : 0.0;
-          a.b_prev = s > 0 ? RKB[s - 1] : 1.0;
-          a.dtpart = T->dtpart;
-        }
-        A(c, a);
-        if (!T->gsur2 || s == 0) B(c, a);
+        a.a = RKA[st];
+        a.b = RKB[st];
+        a.taubar = exact ? T->taubar : nullptr;
+        a.dtpart = exact ? T->dtpart : nullptr;
+        T->ops.launch(c->stream, a, T->afragT);
+        pend = a.gsur;
       }
       if (exact) {
+        // (ubar still lacks stage 0's partner terms; the increments add to it)
         hipLaunchKernelGGL(adjoint_dt_reduce, dim3(1), dim3(256), 0, c->stream, T->dtpart, T->nblk_a, T->clip, n,
                            T->tsc);
         L(c, base, lam, n);
       }
     }
+  }
+  if (pend) {
+    AdjArgs a = adj_args(c);
+    a.gsur = const_cast<double *>(pend);
+    B(c, a);
   }
   HIP_TRY(hipGetLastError());
   const hipMemcpyKind kout = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;

@@ -158,7 +158,7 @@ int dglm_create_from_dir(const dglm_params *p, const char *datain_dir, int matri
 int dglm_destroy(dglm_ctx *ctx);
 
 int dglm_sizes(const dglm_ctx *ctx, int *K, int *Np, int *Nfp, int *nvar);
-/* u: host [nvar][K*Np].  Setting the state zeroes the LSRK register k. */
+/* u: host [nvar][K*Np]. */
 int dglm_set_state(dglm_ctx *ctx, const double *u);
 int dglm_get_state(dglm_ctx *ctx, double *u);
 /* Device-pointer variants (same layout) for callers that own HBM buffers. */
@@ -267,7 +267,9 @@ int dglm_get_timing(dglm_ctx *ctx, double *ms, long *count, int n);
  * ([K*4], optional) = dR/dtau^T rbar per face side.  Host arrays. */
 int dglm_adjoint_rhs(dglm_ctx *ctx, const double *u, const double *rbar, double *ubar, double *taubar);
 /* Advance nsteps from the current state like dglm_step, keeping a checkpoint
- * every `every` steps (sqrt(nsteps) balances memory and recompute). */
+ * every `every` steps (sqrt(nsteps) balances memory and recompute).  Advection
+ * is linear: its reverse sweep needs no states, so nothing is kept or recomputed
+ * there, whatever `every` and dglm_adjoint_set_keep say. */
 int dglm_adjoint_record(dglm_ctx *ctx, int nsteps, int every);
 /* Reverse sweep over the recorded steps: ubar_0 = (du_T/du_0)^T ubar_T.
  * device_ptrs != 0: both pointers are device memory ([nvar][K*Np]).

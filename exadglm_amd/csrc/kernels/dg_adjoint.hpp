@@ -130,13 +130,7 @@ __global__ __launch_bounds__(4 * lam_adj_elems(Ord<N>::Np)) void lambda_adjoint_
   for (int i = t; i < 4 * Nfp; i += NT) s_fm[i] = fmx[((i / Nfp) * 4 + 3) * Nfp + i % Nfp];
   for (int i = t; i < ne * Np; i += NT) {
     const size_t idx = (size_t)e0 * Np + i;
-    const double u1 = u[idx], u2 = u[KNp + idx], u3 = u[2 * KNp + idx], u4 = u[3 * KNp + idx],
-                 u5 = u[4 * KNp + idx];
-    const double vx = u2 / u1, vy = u3 / u1, vz = u4 / u1;
-    const double v2 = vx * vx + vy * vy + vz * vz;
-    const double pres = (gamma - 1.0) * (u5 - 0.5 * u1 * v2);
-    s_v2[i] = v2;
-    s_c2[i] = fabs(gamma * pres / u1);
+    node_speeds(u[idx], u[KNp + idx], u[2 * KNp + idx], u[3 * KNp + idx], u[4 * KNp + idx], gamma, s_v2[i], s_c2[i]);
   }
   __syncthreads();
   const int el = t >> 2, f = t & 3, e = e0 + el;

@@ -277,6 +277,8 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   __shared__ int s_dm[EB * 4];
   __shared__ int s_fmx[16 * Nfp];
 
+  double dt = 0.0;
+  const bool active = MODE == 1 || begin_stage(a, dt);
   const int batch = xcd_batch(order, nbatch);
   if (batch < 0) return;
   const int e0 = batch * EB;
@@ -287,13 +289,12 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t n0 = (size_t)e0 * Np;
 
-  if (MODE == 0 && !a.scal->active) {
+  if (!active) {
     // Past tmax: the stage is the identity on u (k untouched).
     for (int v = 0; v < NV; v++)
       for (int i = tid; i < ne * Np; i += NT) a.u_out[v * KNp + n0 + i] = a.u_in[v * KNp + n0 + i];
     return;
   }
-  const double dt = MODE == 0 ? a.scal->dt : 0.0;
 
   // ---- 1. stage in.  Elements past the end of a short batch get a state at
   // rest and no geometry; their columns are computed and not written ----
@@ -632,13 +633,56 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
         } else {
           const vec kn = a.rka * kr[r] + dt * rhs;
           if (a.k_out) *reinterpret_cast<vec *>(a.k + gi) = kn;
-          *reinterpret_cast<vec *>(a.u_out + gi) = *reinterpret_cast<const vec *>(&s_u[o]) + a.rkb * kn;
+          const vec u1 = *reinterpret_cast<const vec *>(&s_u[o]) + a.rkb * kn;
+          *reinterpret_cast<vec *>(a.u_out + gi) = u1;
+          if (EUL && a.lam_out) *reinterpret_cast<vec *>(&s_u[o]) = u1;
         }
       }
     }
   };
 
   cols_dispatch<S, 0>(w, body);
+
+  // ---- wave speeds of the new state, in a step's last stage: the state is at
+  // hand in LDS, a wave-speed kernel would read it all again ----
+  if constexpr (EUL && MODE == 0) {
+    if (!a.lam_out) return;
+    lds_barrier();
+    for (int i = tid; i < ne * Np; i += NT) {
+      const int e = i / Np, o = e * NS + i - e * Np;
+      node_speeds(s_u[o], s_u[EB * NS + o], s_u[2 * EB * NS + o], s_u[3 * EB * NS + o], s_u[4 * EB * NS + o], a.gamma,
+                  s_x[o], s_x[EB * NS + o]);
+    }
+    lds_barrier();
+    // four threads per face
+    double lfs = 0.0;
+    for (int f0 = 0; f0 < 4 * ne; f0 += NT / 4) {
+      const int fi = f0 + (tid >> 2), e = fi >> 2, f = fi & 3;
+      double mv2 = 0.0, mc2 = 0.0;
+      if (fi < 4 * ne) {
+        for (int j = tid & 3; j < Nfp; j += 4) {
+          const int o = e * NS + s_fmx[(f * 4 + 3) * Nfp + j];
+          const double v2 = s_x[o], c2 = s_x[EB * NS + o];
+          mv2 = v2 > mv2 ? v2 : mv2;
+          mc2 = c2 > mc2 ? c2 : mc2;
+        }
+      }
+#pragma unroll
+      for (int q = 1; q <= 2; q <<= 1) {
+        mv2 = fmax(mv2, __shfl_xor(mv2, q, 64));
+        mc2 = fmax(mc2, __shfl_xor(mc2, q, 64));
+      }
+      if (fi < 4 * ne && (tid & 3) == 0) {
+        const double lam = sqrt(mv2) + sqrt(mc2);
+        a.lam_out[(size_t)e0 * 4 + fi] = lam;
+        double x = lam * s_geo[e * GEO_STRIDE + 9 + f * 4 + 3];
+        // (a non-finite state reaches dt as an infinite wave speed)
+        if (x != x) x = INFINITY;
+        lfs = fmax(lfs, x);
+      }
+    }
+    raise_maxfs(a.clk_out, lfs, s_tau);
+  }
 }
 
 // Elements per workgroup and waves: a large and a small configuration of each

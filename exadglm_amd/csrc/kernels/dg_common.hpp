@@ -14,9 +14,6 @@ struct Ord {
   static constexpr int KD = 3 * Np + NFF;  // stacked contraction length [WDr|WDs|WDt|LIFT]
 };
 
-// Per-step scalars that live in device memory so the step loop never reads
-// back to the host (the reference copies dt to the host every step,
-// euler_nopad_dglm.cu:79-96).
 // Reciprocal and square root for dependency chains that bound a kernel (the
 // fused mixed-precision kernel's surface and volume passes; in the adjoint's
 // pass A and the FP64 warp-specialised kernel they were measured no faster): the
@@ -44,17 +41,24 @@ __device__ inline double sqrt_refined(double x) {
   return x > 0.0 ? g : x;
 }
 
-struct DevScalars {
-  double t;        // start time of the current step
-  double t_next;   // time after the current step (= committed time)
-  double dt;       // step size of the current step
-  double maxfs;    // max over faces of lambda * Fscale
-  int tstep;       // completed steps after the current one
-  int active;      // 0 once t_next >= tmax: stage kernels become no-ops
-  int bad;         // non-finite dt seen
-  int fstar;       // face attaining max(lambda * Fscale) (smallest index on ties)
-  int clipped;     // 1 if dt of the current step was clipped to end at tmax
-  int pad;
+// The step scalars live in device memory, so the step loop never reads back to
+// the host (the reference copies dt to the host every step,
+// euler_nopad_dglm.cu:79-96), in two slots that the steps use in turn: the first
+// stage of a step forms dt from one for itself, leaves it there for the other
+// stages and starts the next step's in the other slot.
+constexpr int MAXFS_SLOTS = 16, MAXFS_STRIDE = 8;  // 64 bytes apart
+struct DevClock {
+  double t;        // start of the step (= the committed time)
+  double dt;       // its size (written by its first stage)
+  double last_dt;  // size of the step before (0: it was past tmax)
+  int active;      // 0: the step is past tmax (written by its first stage)
+  int tstep;       // steps taken
+  int bad;         // a non-finite or non-positive dt was seen
+  int pad[5];
+  // Largest lambda * Fscale over the faces, in parts by workgroup: bits of
+  // doubles >= 0, which order as integers.  One address for the whole grid's
+  // atomics took the wave-speed kernel from 10 to 27 us at 697 workgroups.
+  unsigned long long maxfs[MAXFS_SLOTS * MAXFS_STRIDE];
 };
 
 // Per-element geometry record: 9 metrics followed by 4x(nx,ny,nz,Fscale).
@@ -67,11 +71,33 @@ __host__ __device__ inline int conn_nbr(int c) { return c >> 4; }
 __host__ __device__ inline int conn_face(int c) { return (c >> 2) & 3; }
 __host__ __device__ inline int conn_code(int c) { return c & 3; }
 
-struct PhysParams {
-  double gamma;
-  double tau_scale;
-  double cfl_fac;  // CFL / (2N+1)
-  double tmax;
-};
+// The step that starts at t: dt = CFL/(2N+1) / max(lambda*Fscale), clipped so that
+// the run ends exactly at tmax (euler_time.cpp:49-57); false past tmax.
+__device__ inline bool step_dt(double t, double maxfs, double cfl_fac, double tmax, double &dt, bool &clipped) {
+#pragma clang fp contract(off)
+  dt = 0.0;
+  clipped = false;
+  if (!(t < tmax)) return false;
+  dt = cfl_fac * (1.0 / maxfs);
+  const double end = t + dt;
+  if (end > tmax) {
+    dt = tmax - t;
+    clipped = true;
+  }
+  return true;
+}
+
+// Raise the workgroup's part of maxfs to its largest x >= 0.  red: LDS, one
+// double per wave (at most 16 waves); every thread of the workgroup calls it.
+__device__ inline void raise_maxfs(DevClock *c, double x, double *red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (unsigned w = 1; w < blockDim.x >> 6; w++) x = fmax(x, red[w]);
+    atomicMax(&c->maxfs[blockIdx.x % MAXFS_SLOTS * MAXFS_STRIDE], (unsigned long long)__double_as_longlong(x));
+  }
+}
 
 }  // namespace dglm

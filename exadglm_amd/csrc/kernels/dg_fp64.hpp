@@ -112,7 +112,18 @@ struct StageArgs {
   const int *fmx;
   const double *op;   // [KD][Np]: WDr^T, WDs^T, WDt^T, -LIFT^T
   const double *maxv;
-  const DevScalars *scal;
+  // step clock (device): this step's slot, the next step's (first stage of a step
+  // only: it is started there, its maxfs cleared unless keep_maxfs), and where
+  // dt of this step is recorded (first stage, may be null)
+  DevClock *clk;
+  DevClock *clk_next;
+  double *dt_rec;
+  int keep_maxfs;
+  double cfl_fac, tmax;
+  // the last stage of a step may leave the new state's wave speeds per face and
+  // raise the largest lambda*Fscale of clk_out (null: it does not)
+  double *lam_out;
+  DevClock *clk_out;
   // The LSRK register: rka of a step's first stage is 0, so that stage need not
   // read k, and what the last stage would write (k_out = 0) is never read.
   double rka, rkb;
@@ -127,6 +138,56 @@ struct StageArgs {
   const double *gbnd;
   int nd;
 };
+
+// A value that is the same in every lane, in scalar registers.
+__device__ inline double uniform(double x) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u), hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Start of a stage: dt of its step; false past tmax (the stage is then the
+// identity on the state).  In the first stage of a step workgroup 0 also leaves
+// dt for the other stages and starts the next step's clock.
+__device__ inline bool begin_stage(const StageArgs &a, double &dt) {
+  DevClock *c = a.clk, *n = a.clk_next;
+  if (!n) {
+    dt = uniform(c->dt);
+    return __builtin_amdgcn_readfirstlane(c->active);
+  }
+  const int part = threadIdx.x % MAXFS_SLOTS * MAXFS_STRIDE;
+  const double own = __longlong_as_double((long long)c->maxfs[part]);
+  double fs = own;
+#pragma unroll
+  for (int o = MAXFS_SLOTS / 2; o > 0; o >>= 1) fs = fmax(fs, __shfl_xor(fs, o, 64));
+  const double t = c->t;
+  bool clipped;
+  const bool active = step_dt(t, fs, a.cfl_fac, a.tmax, dt, clipped);
+  if (blockIdx.x == 0 && threadIdx.x < MAXFS_SLOTS) {
+    n->maxfs[part] = a.keep_maxfs ? (unsigned long long)__double_as_longlong(own) : 0;
+    if (threadIdx.x == 0) {
+      c->dt = dt;
+      c->active = active;
+      n->t = active ? t + dt : t;
+      n->last_dt = dt;
+      n->tstep = c->tstep + (active ? 1 : 0);
+      n->bad = c->bad || (active && (!(dt > 0.0) || !isfinite(dt)));
+      if (a.dt_rec) *a.dt_rec = dt;
+    }
+  }
+  dt = uniform(dt);
+  return __builtin_amdgcn_readfirstlane(active ? 1 : 0);
+}
+
+// |v|^2 and |gamma p / rho| of a state, the squares of which calc_maxv takes the
+// face maxima (euler_dglm.cpp:6-50).
+__device__ inline void node_speeds(double u1, double u2, double u3, double u4, double u5, double gamma, double &v2,
+                                   double &c2) {
+  const double vx = u2 / u1, vy = u3 / u1, vz = u4 / u1;
+  v2 = vx * vx + vy * vy + vz * vz;
+  const double pres = (gamma - 1.0) * (u5 - 0.5 * u1 * v2);
+  c2 = fabs(gamma * pres / u1);
+}
 
 // Prescribed boundary state of variable v at face node j of Dirichlet slot ds.
 // The LM flux takes it as the face state ub (the reference leaves the branch
@@ -168,7 +229,8 @@ __global__ __launch_bounds__(256) void stage_simple_kernel(StageArgs a) {
   const int ne = min(EB, K - e0);
   const int tid = threadIdx.x;
 
-  if (MODE == 0 && !a.scal->active) {
+  double dt = 0.0;
+  if (MODE == 0 && !begin_stage(a, dt)) {
     // A step past tmax: keep the state (the caller's buffer swap still happens).
     for (int v = 0; v < NV; v++)
       for (int i = tid; i < ne * Np; i += 256) a.u_out[v * KNp + (size_t)e0 * Np + i] = a.u_in[v * KNp + (size_t)e0 * Np + i];
@@ -257,7 +319,6 @@ __global__ __launch_bounds__(256) void stage_simple_kernel(StageArgs a) {
   __syncthreads();
 
   // Contraction rhs_i = sum_k op[k][i] f[k], then the LSRK register update.
-  const double dt = MODE == 0 ? a.scal->dt : 0.0;
   for (int o = tid; o < NV * ne * Np; o += 256) {
     const int v = o / (ne * Np), r = o - v * (ne * Np);
     const int e = r / Np, i = r - e * Np;

@@ -327,12 +327,12 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   const size_t KNp = (size_t)K * Np;
   const T *afrag = (const T *)afrag_v;
 
-  if (MODE == 0 && !a.scal->active) {
+  double dt = 0.0;
+  if (MODE == 0 && !begin_stage(a, dt)) {
     // Past tmax: the stage is the identity on u (k untouched).
     for (size_t i = (size_t)blockIdx.x * NT + tid; i < NV * KNp; i += (size_t)gridDim.x * NT) a.u_out[i] = a.u_in[i];
     return;
   }
-  const double dt = MODE == 0 ? a.scal->dt : 0.0;
 
   // Operator rows of this wave, resident for the whole kernel.
   T afr[BF ? 1 : KS];

@@ -338,12 +338,12 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
   const int K = a.K;
   const size_t KNp = (size_t)K * Np;
 
-  if (MODE == 0 && !a.scal->active) {
+  double dt = 0.0;
+  if (MODE == 0 && !begin_stage(a, dt)) {
     // Past tmax: the stage is the identity on u (k untouched).
     for (size_t i = (size_t)blockIdx.x * NT + tid; i < 5 * KNp; i += (size_t)gridDim.x * NT) a.u_out[i] = a.u_in[i];
     return;
   }
-  const double dt = MODE == 0 ? a.scal->dt : 0.0;
   const double gamma = a.gamma;
 
   for (int i = tid; i < 16 * Nfp; i += NT) s_fmx[i] = a.fmx[i];

@@ -1,19 +1,18 @@
 // Per-step reductions that are plain (non-template) kernels: the device-side
 // dt, its adjoint and the conserved integrals.  Included by solver.hip only, so each is
 // defined in one translation unit.
-//   calc_dt  dim3/src/cpp/euler_dglm.cpp:53-69, euler_time.cpp:49-57
 #pragma once
 #include "dg_common.hpp"
 
 namespace dglm {
 
-// dt = CFL/(2N+1) / max(lambda*Fscale), clipped so the run ends exactly at
-// tmax (euler_time.cpp:49-57).  One block.
-__global__ __launch_bounds__(1024) void finalize_dt_kernel(const double *__restrict__ partial,
-                                                            const int *__restrict__ partial_idx, int n,
-                                                            DevScalars *s, double cfl_fac, double tmax,
-                                                            double *dt_hist, int *fstar_hist, int *clip_hist,
-                                                            int hist_idx) {
+// The adjoint's recording: the largest of the wave-speed blocks' maxima into the
+// step's clock, and its face (smallest index on ties), dt and the clip flag into
+// the step's entries of the tape.  One block.
+__global__ __launch_bounds__(1024) void record_dt_kernel(const double *__restrict__ partial,
+                                                         const int *__restrict__ partial_idx, int n, DevClock *s,
+                                                         double cfl_fac, double tmax, double *dt_rec, int *fstar_rec,
+                                                         int *clip_rec) {
   __shared__ double red[1024];
   __shared__ int red_i[1024];
   double m = 0.0;
@@ -39,31 +38,48 @@ __global__ __launch_bounds__(1024) void finalize_dt_kernel(const double *__restr
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const double maxfs = red[0];
-    const double t = s->t_next;
-    s->maxfs = maxfs;
-    s->fstar = red_i[0];
-    s->clipped = 0;
-    if (t < tmax) {
-      double dt = cfl_fac * (1.0 / maxfs);
-      if (t + dt > tmax) {
-        dt = tmax - t;
-        s->clipped = 1;
-      }
-      s->t = t;
-      s->dt = dt;
-      s->t_next = t + dt;
-      s->tstep += 1;
-      s->active = 1;
-      if (!(dt > 0.0) || !isfinite(dt)) s->bad = 1;
-    } else {
-      s->active = 0;
-      s->dt = 0.0;
-    }
-    if (dt_hist) dt_hist[hist_idx] = s->active ? s->dt : 0.0;
-    if (fstar_hist) fstar_hist[hist_idx] = s->fstar;
-    if (clip_hist) clip_hist[hist_idx] = s->clipped;
+    s->maxfs[0] = (unsigned long long)__double_as_longlong(red[0]);
+    for (int i = 1; i < MAXFS_SLOTS; i++) s->maxfs[i * MAXFS_STRIDE] = 0;
+    double dt;
+    bool clipped;
+    step_dt(s->t, red[0], cfl_fac, tmax, dt, clipped);
+    if (dt_rec) *dt_rec = dt;
+    if (fstar_rec) *fstar_rec = red_i[0];
+    if (clip_rec) *clip_rec = clipped;
   }
+}
+
+// Clock updates between steps: copy *src (when given), set the time (what & 1),
+// clear maxfs (what & 2).  MAXFS_SLOTS threads.
+__global__ void set_clock_kernel(DevClock *c, const DevClock *src, int what, double t, int tstep) {
+  const int part = threadIdx.x * MAXFS_STRIDE;
+  if (src || (what & 2)) c->maxfs[part] = what & 2 ? 0 : src->maxfs[part];
+  if (threadIdx.x != 0) return;
+  if (src) {
+    c->t = src->t;
+    c->last_dt = src->last_dt;
+    c->tstep = src->tstep;
+    c->bad = src->bad;
+  }
+  if (what & 1) {
+    c->t = t;
+    c->last_dt = 0.0;
+    c->tstep = tstep;
+    c->bad = 0;
+  }
+}
+
+struct ClockReport {
+  double t, last_dt;
+  int tstep, bad;
+};
+
+// The clock and the first n dt of a step call into mapped host memory.
+__global__ __launch_bounds__(256) void report_kernel(const DevClock *c, const double *dt_hist, int n,
+                                                     ClockReport *c_out, double *dt_out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dt_out[i] = dt_hist[i];
+  if (i == 0) *c_out = {c->t, c->last_dt, c->tstep, c->bad};
 }
 
 // Conserved integrals sum_e J_e w^T u_e (w = column sums of M), FP64: one

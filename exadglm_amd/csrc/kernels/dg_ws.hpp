@@ -629,12 +629,12 @@ __global__ __launch_bounds__(WsShape<N>::NT) void stage_ws_kernel(StageArgs a, c
   const int w = __builtin_amdgcn_readfirstlane(ws_role<N>(tid >> 6));  // role, uniform: role branches are scalar
   const size_t KNp = (size_t)a.K * Np;
 
-  if (MODE == 0 && !a.scal->active) {
+  double dt = 0.0;
+  if (MODE == 0 && !begin_stage(a, dt)) {
     // Past tmax: the stage is the identity on u (k untouched).
     for (size_t i = (size_t)blockIdx.x * NT + tid; i < 5 * KNp; i += (size_t)gridDim.x * NT) a.u_out[i] = a.u_in[i];
     return;
   }
-  const double dt = MODE == 0 ? a.scal->dt : 0.0;
 
   for (int i = tid; i < 16 * Nfp; i += NT) s_fmx[i] = a.fmx[i];
   for (int i = tid; i < REM * KDP; i += NT) s_arem[i] = arem[i];
@@ -710,8 +710,9 @@ __global__ __launch_bounds__(WsShape<N>::NT) void stage_ws_kernel(StageArgs a, c
 // LDS-staged wave speed: a block converts the node values of WE elements to
 // |v|^2 and |c|^2 with coalesced loads, then one thread per face takes the
 // maxima over the face nodes (calc_maxv, euler_dglm.cpp:6-50,
-// advec_dglm.cpp:6-35); the block keeps the largest lambda*Fscale with its
-// face index (smallest index on ties).
+// advec_dglm.cpp:6-35).  The largest lambda*Fscale goes to the clock;
+// without one the block keeps its own with the face index (smallest index on ties),
+// for the adjoint's recording.
 // --------------------------------------------------------------------------
 __host__ __device__ constexpr int wavespeed_elems(int Np) { return Np <= 35 ? 64 : (Np <= 84 ? 32 : 16); }
 
@@ -720,6 +721,7 @@ __global__ __launch_bounds__(256) void wavespeed_lds_kernel(int K, const double 
                                                             const double *__restrict__ vel,
                                                             const double *__restrict__ geo,
                                                             const int *__restrict__ fmx, double *__restrict__ maxv,
+                                                            DevClock *clk,
                                                             double *__restrict__ partial,
                                                             int *__restrict__ partial_idx, double gamma) {
   using O = Ord<N>;
@@ -737,13 +739,7 @@ __global__ __launch_bounds__(256) void wavespeed_lds_kernel(int K, const double 
   for (int i = tid; i < ne * Np; i += 256) {
     const size_t idx = (size_t)e0 * Np + i;
     if (PHYS == PHYS_EULER) {
-      const double u1 = u[idx], u2 = u[KNp + idx], u3 = u[2 * KNp + idx], u4 = u[3 * KNp + idx],
-                   u5 = u[4 * KNp + idx];
-      const double vx = u2 / u1, vy = u3 / u1, vz = u4 / u1;
-      const double v2 = vx * vx + vy * vy + vz * vz;
-      const double pres = (gamma - 1.0) * (u5 - 0.5 * u1 * v2);
-      s_v2[i] = v2;
-      s_c2[i] = fabs(gamma * pres / u1);
+      node_speeds(u[idx], u[KNp + idx], u[2 * KNp + idx], u[3 * KNp + idx], u[4 * KNp + idx], gamma, s_v2[i], s_c2[i]);
     } else {
       const double vx = vel[idx], vy = vel[KNp + idx], vz = vel[2 * KNp + idx];
       s_v2[i] = vx * vx + vy * vy + vz * vz;
@@ -770,6 +766,10 @@ __global__ __launch_bounds__(256) void wavespeed_lds_kernel(int K, const double 
     // A non-finite state (no maximum over a NaN) reaches dt as an infinite
     // wave speed: dt = 0 is flagged as bad on the device.
     if (lfs != lfs) lfs = INFINITY;
+  }
+  if (clk) {
+    raise_maxfs(clk, lfs, red);
+    return;
   }
   red[tid] = lfs;
   red_i[tid] = tid < ne * 4 ? fid : 0x7fffffff;

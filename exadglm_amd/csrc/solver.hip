@@ -39,7 +39,9 @@ bool launch_ws_dirichlet(int N, int mode, int grid, hipStream_t stream, const St
                          const double *arem, const int *order, int nbatch, int groups);
 }  // namespace dglm
 
-#define DGLM_NTIMERS 3  // wave speed, dt finalize, stage
+#define DGLM_NTIMERS 3  // wave speed, (none), stage
+
+constexpr int REPORT_MAX = 1024;  // steps whose dt a report carries
 
 namespace {
 thread_local std::string g_err;
@@ -77,13 +79,24 @@ struct dglm_ctx {
   int dev = 0;
   hipStream_t stream = nullptr;
   double *u[2] = {nullptr, nullptr};
-  double *k = nullptr, *rhs = nullptr, *vel = nullptr, *geo = nullptr, *op = nullptr, *maxv = nullptr,
+  double *k = nullptr, *rhs = nullptr, *vel = nullptr, *geo = nullptr, *op = nullptr,
          *partial = nullptr, *dt_hist = nullptr;
   double *scratch = nullptr;  // this device's copy of the allocation-free scratch array
   int dt_hist_cap = 0;
   int *conn = nullptr, *fmx = nullptr, *partial_idx = nullptr;
-  DevScalars *scal = nullptr;
+  // The buffer the next step starts from; also the slot of its clock and of its
+  // wave speeds (a step is an odd number of stages: both alternate).  Advection's
+  // wave speeds are constant: both slots are one buffer.
   int cur = 0;
+  DevClock *clk = nullptr;                  // [2]
+  double *maxv[2] = {nullptr, nullptr};     // wave speeds per face
+  bool lam_ok = false;                      // maxv[cur] and clk[cur].maxfs are those of u[cur]
+  // Mapped host memory that the device reports the clock and dt histories of up
+  // to REPORT_MAX steps into (pageable copies cost 20-30 us each).
+  struct HostReport {
+    ClockReport clk;
+    double dt[REPORT_MAX];
+  } *h_rep = nullptr;
   int nblk_ws = 0;
   int variant = DGLM_STAGE_AUTO;  // requested stage kernel
   void *afrag = nullptr;          // operator A-fragments of the mixed-precision MFMA kernel
@@ -266,13 +279,13 @@ extern "C" int dglm_mesh_spatial_h(int K, const int *EtoV, const double *VXYZ, d
 // ---------------------------------------------------------------------------
 namespace {
 
-// Wave speed of state u into maxv, with the per-block maxima of lambda*Fscale
-// (and their face indices) in partial / partial_idx [nblk_ws] for the dt
-// kernel.
+// Wave speed of state u into maxv, and the largest lambda*Fscale into the clock; without
+// one the per-block maxima and their face indices in the context's partial
+// buffers [nblk_ws].
 template <int N, int PHYS>
-void launch_wavespeed(dglm_ctx *c, const double *u, double *maxv, double *partial, int *partial_idx) {
+void launch_wavespeed(dglm_ctx *c, const double *u, double *maxv, DevClock *clk) {
   hipLaunchKernelGGL((wavespeed_lds_kernel<N, PHYS>), dim3(c->nblk_ws), dim3(256), 0, c->stream, c->K, u, c->vel,
-                     c->geo, c->fmx, maxv, partial, partial_idx, c->p.gamma);
+                     c->geo, c->fmx, maxv, clk, c->partial, c->partial_idx, c->p.gamma);
 }
 
 // True when the MFMA stage kernel can be selected for this order (above it the
@@ -411,7 +424,7 @@ void launch_stage(dglm_ctx *c, const StageArgs &a) {
   }
 }
 
-typedef void (*ws_fn)(dglm_ctx *, const double *, double *, double *, int *);
+typedef void (*ws_fn)(dglm_ctx *, const double *, double *, DevClock *);
 typedef void (*st_fn)(dglm_ctx *, const StageArgs &);
 
 template <int PHYS>
@@ -456,8 +469,9 @@ StageArgs stage_args(dglm_ctx *c, int s) {
   a.conn = c->conn;
   a.fmx = c->fmx;
   a.op = c->op;
-  a.maxv = c->maxv;
-  a.scal = c->scal;
+  a.maxv = c->maxv[c->cur];
+  a.cfl_fac = c->p.cfl / (2 * c->p.N + 1);
+  a.tmax = c->p.tmax;
   a.rka = s >= 0 ? RKA[s] : 0.0;
   a.rkb = s >= 0 ? RKB[s] : 0.0;
   a.k_out = s != 4;
@@ -494,11 +508,13 @@ void free_ctx(dglm_ctx *c) {
   if (!c) return;
   hipSetDevice(c->dev);
   if (c->stream) hipStreamSynchronize(c->stream);
-  void *ptrs[] = {c->u[0], c->u[1], c->k, c->rhs, c->vel, c->geo, c->op, c->maxv, c->partial, c->dt_hist,
-                  c->conn, c->fmx, c->scal, c->afrag, c->rowsum, c->partial_idx, c->afrag_ws, c->arem_ws,
+  void *ptrs[] = {c->u[0], c->u[1], c->k, c->rhs, c->vel, c->geo, c->op, c->maxv[0],
+                  c->maxv[1] != c->maxv[0] ? c->maxv[1] : nullptr, c->partial, c->dt_hist,
+                  c->conn, c->fmx, c->clk, c->afrag, c->rowsum, c->partial_idx, c->afrag_ws, c->arem_ws,
                   c->ws_order, c->dmap, c->gbnd, c->mx_tab, c->afrag_cols, c->cols_order};
   for (void *q : ptrs)
     if (q) hipFree(q);
+  if (c->h_rep) hipHostFree(c->h_rep);
   free_tape(c->tape);
   for (int g = 0; g < 2; g++)
     if (c->graph[g]) hipGraphExecDestroy(c->graph[g]);
@@ -824,11 +840,12 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   const size_t nst = (size_t)c->nvar * K * Np;
   if ((rc = dev_alloc(&c->u[0], nst, "u0")) || (rc = dev_alloc(&c->u[1], nst, "u1")) ||
       (rc = dev_alloc(&c->k, nst, "k")) || (rc = dev_alloc(&c->geo, geo.size(), "geo")) ||
-      (rc = dev_alloc(&c->op, op.size(), "op")) || (rc = dev_alloc(&c->maxv, (size_t)K * 4, "maxv")) ||
+      (rc = dev_alloc(&c->op, op.size(), "op")) || (rc = dev_alloc(&c->maxv[0], (size_t)K * 4, "maxv")) ||
+      (c->nvar == 5 && (rc = dev_alloc(&c->maxv[1], (size_t)K * 4, "maxv"))) ||
       (rc = dev_alloc(&c->partial, (size_t)c->nblk_ws, "partial")) ||
       (rc = dev_alloc(&c->partial_idx, (size_t)c->nblk_ws, "partial index")) ||
       (rc = dev_alloc(&c->conn, conn.size(), "conn")) || (rc = dev_alloc(&c->fmx, fmx.size(), "fmx")) ||
-      (rc = dev_alloc(&c->scal, 1, "scalars")) ||
+      (rc = dev_alloc(&c->clk, 2, "step clock")) ||
       (afrag_bytes && (rc = dev_alloc((char **)&c->afrag, afrag_bytes, "A-fragments"))) ||
       (!afr_ws.empty() && (rc = dev_alloc(&c->afrag_ws, afr_ws.size(), "A-fragments (warp-specialised)"))) ||
       (!arem_ws.empty() && (rc = dev_alloc(&c->arem_ws, arem_ws.size(), "remainder rows"))) ||
@@ -854,8 +871,12 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
     free_ctx(c);
     return fail(DGLM_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(he));
   }
-  DevScalars s0{};
-  s0.active = 1;
+  if (c->nvar == 1) c->maxv[1] = c->maxv[0];
+  he = hipHostMalloc((void **)&c->h_rep, sizeof(*c->h_rep), hipHostMallocMapped);
+  if (he != hipSuccess) {
+    free_ctx(c);
+    return fail(DGLM_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(he));
+  }
   hipError_t errs[] = {
       hipMemcpy(c->geo, geo.data(), geo.size() * sizeof(double), hipMemcpyHostToDevice),
       hipMemcpy(c->op, op.data(), op.size() * sizeof(double), hipMemcpyHostToDevice),
@@ -877,7 +898,7 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
                 : hipSuccess,
       c->dmap ? hipMemcpy(c->dmap, dmap.data(), dmap.size() * sizeof(int), hipMemcpyHostToDevice) : hipSuccess,
       c->mx_tab ? hipMemcpy(c->mx_tab, mx_tab.data(), mx_tab.size(), hipMemcpyHostToDevice) : hipSuccess,
-      hipMemcpy(c->scal, &s0, sizeof(s0), hipMemcpyHostToDevice),
+      hipMemset(c->clk, 0, 2 * sizeof(DevClock)),
       hipMemset(c->u[0], 0, nst * sizeof(double)),
       hipMemset(c->u[1], 0, nst * sizeof(double)),
   };
@@ -941,11 +962,23 @@ extern "C" int dglm_sizes(const dglm_ctx *c, int *K, int *Np, int *Nfp, int *nva
   return DGLM_OK;
 }
 
+// The wave speeds on the device are no longer those of the state (advection's
+// depend on the velocity alone).
+static void stale_speeds(dglm_ctx *c, bool velocity = false) {
+  if (c->nvar == 1 && !velocity) return;
+  c->lam_ok = false;
+  hipLaunchKernelGGL(set_clock_kernel, dim3(1), dim3(MAXFS_SLOTS), 0, c->stream, c->clk + c->cur, (const DevClock *)nullptr, 2,
+                     0.0, 0);
+}
+
 static int set_state_impl(dglm_ctx *c, const double *u, hipMemcpyKind kind) {
   if (!c || !u) return fail(DGLM_ERR_ARG, "dglm_set_state: null argument");
   HIP_TRY(hipSetDevice(c->dev));
   const size_t n = (size_t)c->nvar * c->K * c->Np;
+  if (c->cur != 0)  // the clock goes with the buffer
+    hipLaunchKernelGGL(set_clock_kernel, dim3(1), dim3(MAXFS_SLOTS), 0, c->stream, c->clk, c->clk + 1, 0, 0.0, 0);
   c->cur = 0;
+  stale_speeds(c);
   HIP_TRY(hipMemcpyAsync(c->u[0], u, n * sizeof(double), kind, c->stream));
   // (the LSRK register needs no clearing: a step's first stage does not read it)
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -976,9 +1009,12 @@ extern "C" int dglm_set_velocity(dglm_ctx *c, const double *vx, const double *vy
   if (!c->vel) return fail(DGLM_ERR_ARG, "dglm_set_velocity: only for advection");
   HIP_TRY(hipSetDevice(c->dev));
   const size_t n = (size_t)c->K * c->Np;
+  HIP_TRY(hipStreamSynchronize(c->stream));
   HIP_TRY(hipMemcpy(c->vel, vx, n * sizeof(double), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->vel + n, vy, n * sizeof(double), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->vel + 2 * n, vz, n * sizeof(double), hipMemcpyHostToDevice));
+  stale_speeds(c, true);
+  HIP_TRY(hipGetLastError());
   return DGLM_OK;
 }
 
@@ -1019,12 +1055,23 @@ static int need_dirichlet(const dglm_ctx *c, const char *who) {
 extern "C" int dglm_set_time(dglm_ctx *c, double t, int tstep) {
   if (!c) return fail(DGLM_ERR_ARG, "dglm_set_time: null context");
   HIP_TRY(hipSetDevice(c->dev));
-  DevScalars s{};
-  s.t = t;
-  s.t_next = t;
-  s.tstep = tstep;
-  s.active = 1;
-  HIP_TRY(hipMemcpyAsync(c->scal, &s, sizeof(s), hipMemcpyHostToDevice, c->stream));
+  // (the step past tmax leaves no wave speeds of the new state: form them anew)
+  hipLaunchKernelGGL(set_clock_kernel, dim3(1), dim3(MAXFS_SLOTS), 0, c->stream, c->clk + c->cur, (const DevClock *)nullptr, 1,
+                     t, tstep);
+  stale_speeds(c);
+  HIP_TRY(hipGetLastError());
+  return DGLM_OK;
+}
+
+// The clock of the next step (and the first n entries of a dt history) into the
+// mapped host memory; synchronises.
+static int report(dglm_ctx *c, const double *hist, int n) {
+  void *d = nullptr;
+  HIP_TRY(hipHostGetDevicePointer(&d, c->h_rep, 0));
+  dglm_ctx::HostReport *out = (dglm_ctx::HostReport *)d;
+  hipLaunchKernelGGL(report_kernel, dim3(n / 256 + 1), dim3(256), 0, c->stream, c->clk + c->cur, hist, n,
+                     &out->clk, out->dt);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(c->stream));
   return DGLM_OK;
 }
@@ -1032,13 +1079,12 @@ extern "C" int dglm_set_time(dglm_ctx *c, double t, int tstep) {
 extern "C" int dglm_get_time(dglm_ctx *c, double *t, double *dt, int *tstep, int *done) {
   if (!c) return fail(DGLM_ERR_ARG, "dglm_get_time: null context");
   HIP_TRY(hipSetDevice(c->dev));
-  DevScalars s;
-  HIP_TRY(hipMemcpyAsync(&s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  if (t) *t = s.t_next;
-  if (dt) *dt = s.dt;
+  if (int rc = report(c, nullptr, 0)) return rc;
+  const ClockReport s = c->h_rep->clk;
+  if (t) *t = s.t;
+  if (dt) *dt = s.last_dt;
   if (tstep) *tstep = s.tstep;
-  if (done) *done = !(s.t_next < c->p.tmax);
+  if (done) *done = !(s.t < c->p.tmax);
   if (s.bad) return fail(DGLM_ERR_STATE, "non-finite or non-positive dt encountered (state diverged)");
   return DGLM_OK;
 }
@@ -1055,8 +1101,9 @@ extern "C" int dglm_rhs(dglm_ctx *c, const double *u, double *rhs, double *maxv,
     int rc = dev_alloc(&c->rhs, n, "rhs");
     if (rc) return rc;
   }
+  stale_speeds(c);  // (u goes into the step's buffer)
   HIP_TRY(hipMemcpyAsync(c->u[c->cur], u, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  ws(c, c->u[c->cur], c->maxv, c->partial, c->partial_idx);
+  ws(c, c->u[c->cur], c->maxv[c->cur], nullptr);
   StageArgs a = stage_args(c, -1);
   st1(c, a);
   HIP_TRY(hipGetLastError());
@@ -1064,7 +1111,7 @@ extern "C" int dglm_rhs(dglm_ctx *c, const double *u, double *rhs, double *maxv,
   std::vector<double> lam;
   if (maxv || tau) {
     lam.resize((size_t)c->K * 4);
-    HIP_TRY(hipMemcpyAsync(lam.data(), c->maxv, lam.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(lam.data(), c->maxv[c->cur], lam.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (maxv) memcpy(maxv, lam.data(), lam.size() * sizeof(double));
@@ -1077,27 +1124,49 @@ extern "C" int dglm_rhs(dglm_ctx *c, const double *u, double *rhs, double *maxv,
 }
 
 namespace {
-// One LSRK4(5) step: wave speed, device-side dt, five fused stages.  The
-// wave-speed block maxima go through partial / partial_idx [nblk_ws]; dt_hist
-// (device, optional) receives dt at hist_idx.  timed: per-kernel HIP events
-// when the context's timing is on.
-void enqueue_step(dglm_ctx *c, ws_fn ws, st_fn st0, double *dt_hist, int hist_idx, double *partial,
-                  int *partial_idx, bool timed = true) {
-  const double cfl_fac = c->p.cfl / (2 * c->p.N + 1);
-  int tk = timed ? timer_start(c, 0) : -1;
-  ws(c, c->u[c->cur], c->maxv, partial, partial_idx);
-  timer_stop(c, tk);
-  tk = timed ? timer_start(c, 1) : -1;
-  hipLaunchKernelGGL(finalize_dt_kernel, dim3(1), dim3(1024), 0, c->stream, partial, partial_idx, c->nblk_ws,
-                     c->scal, cfl_fac, c->p.tmax, dt_hist, (int *)nullptr, (int *)nullptr, hist_idx);
-  timer_stop(c, tk);
+// Whether a step leaves the wave speeds of its new state: advection's are
+// constant, and the packed-column kernel's last Euler stage forms them on meshes
+// of few batches, where the separate kernel costs mostly its launch (a step at
+// N = 4, K = 384: 46 -> 39 us; N = 5, K = 1296: 70 -> 62).  On larger ones its two
+// barriers at the end of every workgroup cost more than the kernel (N = 3, K =
+// 44,574: 8 us a step more, N = 4, K = 11,520: 3).
+constexpr int LEAVE_SPEEDS_MAX_BATCHES = 2048;
+bool step_leaves_speeds(const dglm_ctx *c) {
+  if (c->nvar == 1) return true;
+  return c->p.precision == DGLM_FP64 && (stage_kind(c) == DGLM_STAGE_MFMA || c->p.N > 6) &&
+         (c->K + c->cols.eb - 1) / c->cols.eb <= LEAVE_SPEEDS_MAX_BATCHES;
+}
+
+// One LSRK4(5) step: the wave speed where the step before did not leave it, five
+// fused stages.  dt_rec (device, optional) receives dt.  timed: per-kernel HIP
+// events when the context's timing is on.
+void enqueue_step(dglm_ctx *c, ws_fn ws, st_fn st0, double *dt_rec, bool timed = true) {
+  const int p = c->cur;
+  const bool leaves = step_leaves_speeds(c);
+  if (!c->lam_ok) {
+    int tk = timed ? timer_start(c, 0) : -1;
+    ws(c, c->u[p], c->maxv[p], c->clk + p);
+    timer_stop(c, tk);
+  }
   for (int s = 0; s < 5; s++) {
     StageArgs a = stage_args(c, s);
-    tk = timed ? timer_start(c, 2) : -1;
+    a.maxv = c->maxv[p];
+    a.clk = c->clk + p;
+    if (s == 0) {
+      a.clk_next = c->clk + (p ^ 1);
+      a.dt_rec = dt_rec;
+      a.keep_maxfs = c->nvar == 1;
+    }
+    if (s == 4 && leaves && c->nvar == 5) {
+      a.lam_out = c->maxv[p ^ 1];
+      a.clk_out = c->clk + (p ^ 1);
+    }
+    int tk = timed ? timer_start(c, 2) : -1;
     st0(c, a);
     timer_stop(c, tk);
     c->cur ^= 1;
   }
+  c->lam_ok = leaves;
 }
 
 void drop_graphs(dglm_ctx *c) {
@@ -1114,8 +1183,8 @@ int build_graph(dglm_ctx *c, ws_fn ws, st_fn st0) {
   const int start = c->cur;
   hipGraph_t g = nullptr;
   HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  enqueue_step(c, ws, st0, nullptr, 0, c->partial, c->partial_idx);
-  enqueue_step(c, ws, st0, nullptr, 0, c->partial, c->partial_idx);
+  enqueue_step(c, ws, st0, nullptr);
+  enqueue_step(c, ws, st0, nullptr);
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   c->cur = start;
   if (e != hipSuccess) return fail(DGLM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
@@ -1128,6 +1197,18 @@ int build_graph(dglm_ctx *c, ws_fn ws, st_fn st0) {
   return DGLM_OK;
 }
 }  // namespace
+
+// A step call's dt history from the device.
+static int fetch_dt(dglm_ctx *c, const double *d_hist, int nsteps, double *dt_hist) {
+  if (nsteps <= REPORT_MAX) {
+    if (int rc = report(c, d_hist, nsteps)) return rc;
+    memcpy(dt_hist, c->h_rep->dt, (size_t)nsteps * sizeof(double));
+    return DGLM_OK;
+  }
+  HIP_TRY(hipMemcpyAsync(dt_hist, d_hist, (size_t)nsteps * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return DGLM_OK;
+}
 
 extern "C" int dglm_step(dglm_ctx *c, int nsteps, double *dt_hist) {
   if (!c || nsteps < 0) return fail(DGLM_ERR_ARG, "dglm_step: bad arguments");
@@ -1149,8 +1230,10 @@ extern "C" int dglm_step(dglm_ctx *c, int nsteps, double *dt_hist) {
   // fixed before capture.
   const bool graphs = c->use_graph && !dt_hist && !c->timing;
   if (graphs && nsteps >= 3) {
-    if (!c->graph[c->cur ^ 1] && !c->graph[c->cur]) {
-      enqueue_step(c, ws, st0, nullptr, 0, c->partial, c->partial_idx);
+    // (the captured steps begin with or without a wave-speed kernel: a step
+    // that has to begin the other way runs eagerly too)
+    if ((!c->graph[c->cur ^ 1] && !c->graph[c->cur]) || c->lam_ok != step_leaves_speeds(c)) {
+      enqueue_step(c, ws, st0, nullptr);
       st++;
     }
     while (nsteps - st >= 2) {
@@ -1163,17 +1246,14 @@ extern "C" int dglm_step(dglm_ctx *c, int nsteps, double *dt_hist) {
     }
   }
   for (; st < nsteps; st++) {
-    enqueue_step(c, ws, st0, dt_hist ? c->dt_hist : nullptr, st, c->partial, c->partial_idx);
+    enqueue_step(c, ws, st0, dt_hist ? c->dt_hist + st : nullptr);
     if (c->ev_class.size() > 8192) {
       int rc = timer_flush(c);
       if (rc) return rc;
     }
   }
   HIP_TRY(hipGetLastError());
-  if (dt_hist) {
-    HIP_TRY(hipMemcpyAsync(dt_hist, c->dt_hist, (size_t)nsteps * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  }
+  if (dt_hist) return fetch_dt(c, c->dt_hist, nsteps, dt_hist);
   return DGLM_OK;
 }
 
@@ -1192,18 +1272,11 @@ extern "C" int dglm_step_noalloc(dglm_ctx *c, int nsteps, double *dt_hist) {
   st_fn st0, st1;
   if (!dispatch(c, ws, st0, st1)) return fail(DGLM_ERR_UNSUPPORTED, "dglm_step_noalloc: order not built");
   HIP_TRY(hipSetDevice(c->dev));
-  // Every scratch entry a step reads is written earlier in the same step
-  // (block maxima by the wave-speed kernel, dt by the dt kernel), so nothing
-  // left by an earlier call is read and nothing needs clearing.
+  // The dt history is the only scratch: every entry read is written by this call.
   double *hist = c->scratch;
-  double *part = c->scratch + DGLM_NOALLOC_MAX_STEPS;
-  int *pidx = (int *)(part + DGLM_NOALLOC_MAX_BLOCKS);
-  for (int st = 0; st < nsteps; st++) enqueue_step(c, ws, st0, dt_hist ? hist : nullptr, st, part, pidx, false);
+  for (int st = 0; st < nsteps; st++) enqueue_step(c, ws, st0, dt_hist ? hist + st : nullptr, false);
   HIP_TRY(hipGetLastError());
-  if (dt_hist) {
-    HIP_TRY(hipMemcpyAsync(dt_hist, hist, (size_t)nsteps * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  }
+  if (dt_hist) return fetch_dt(c, hist, nsteps, dt_hist);
   return DGLM_OK;
 }
 
@@ -1354,14 +1427,17 @@ bool adj_dispatch(const dglm_ctx *c, adj_fn &B, lam_fn &Lf) {
   return c->p.physics == DGLM_EULER ? pick_adj<PHYS_EULER>(c->p.N, B, Lf) : pick_adj<PHYS_ADV>(c->p.N, B, Lf);
 }
 
-StageArgs make_stage_args(dglm_ctx *c, const double *u_in, double *u_out, double *k, const double *maxv,
-                          const DevScalars *scal, int s) {
+// A stage of a step on clock slot q of clk[2] (the adjoint's recording and
+// recompute: states and wave speeds where the tape wants them).
+StageArgs make_stage_args(dglm_ctx *c, const double *u_in, double *u_out, double *k, const double *maxv, DevClock *clk,
+                          int q, int s) {
   StageArgs a = stage_args(c, s);
   a.u_in = u_in;
   a.u_out = u_out;
   a.k = k;
   a.maxv = maxv;
-  a.scal = scal;
+  a.clk = clk + q;
+  a.clk_next = s == 0 ? clk + (q ^ 1) : nullptr;
   return a;
 }
 
@@ -1374,7 +1450,7 @@ struct dglm_adj_tape {
   int *order = nullptr;      // its batch visiting order (null: mesh order)
   double *ckpt = nullptr, *ck_t = nullptr, *dt = nullptr, *seg = nullptr, *lam = nullptr, *kscr = nullptr;
   int *fstar = nullptr, *clip = nullptr, *ck_step = nullptr;
-  DevScalars *scal2 = nullptr;
+  DevClock *clk2 = nullptr;  // [2], the recompute's step clock
   double *ubar = nullptr, *kbar = nullptr, *gsur = nullptr, *taubar = nullptr, *dtpart = nullptr, *tsc = nullptr;
   // second face-term buffer: each pass A reads the terms of the one before it
   // while writing its own
@@ -1402,7 +1478,7 @@ void launch_lam(dglm_ctx *c, const double *u, const double *lam, int step) {
 
 void free_tape(dglm_adj_tape *T) {
   if (!T) return;
-  void *ptrs[] = {T->keep, T->keep_lam, T->ckpt, T->ck_t, T->dt, T->seg, T->lam, T->kscr, T->fstar, T->clip, T->ck_step, T->scal2,
+  void *ptrs[] = {T->keep, T->keep_lam, T->ckpt, T->ck_t, T->dt, T->seg, T->lam, T->kscr, T->fstar, T->clip, T->ck_step, T->clk2,
                   T->ubar, T->kbar, T->gsur, T->gsur2, T->taubar, T->dtpart, T->tsc, T->rbar, T->slots, T->pslot,
                   T->afragT, T->order};
   for (void *q : ptrs)
@@ -1502,14 +1578,15 @@ extern "C" int dglm_adjoint_rhs(dglm_ctx *c, const double *u, const double *rbar
   lam_fn L;
   if (!dispatch(c, ws, st0, st1) || !adj_dispatch(c, B, L))
     return fail(DGLM_ERR_UNSUPPORTED, "dglm_adjoint_rhs: order not built");
+  stale_speeds(c);  // (u goes into the step's buffer)
   HIP_TRY(hipMemcpyAsync(c->u[c->cur], u, nst * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipMemcpyAsync(T->rbar, rbar, nst * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  ws(c, c->u[c->cur], c->maxv, c->partial, c->partial_idx);  // tau at u
+  ws(c, c->u[c->cur], c->maxv[c->cur], nullptr);  // tau at u
   AdjArgs a = adj_args(c);
   a.mode = 1;
   a.u = c->u[c->cur];
   a.rbar = T->rbar;
-  a.maxv = c->maxv;
+  a.maxv = c->maxv[c->cur];
   T->ops.launch(c->stream, a, T->afragT);
   B(c, a);
   HIP_TRY(hipGetLastError());
@@ -1546,8 +1623,8 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
       T->nsteps = nsteps;
       T->bytes = T->base_bytes + ((size_t)c->K * 4 + nsteps) * sizeof(double);
     }
-    for (int n = 0; n < nsteps; n++) enqueue_step(c, ws, st0, T->dt, n, c->partial, c->partial_idx, false);
-    HIP_TRY(hipMemcpyAsync(T->lam, c->maxv, (size_t)c->K * 4 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    for (int n = 0; n < nsteps; n++) enqueue_step(c, ws, st0, T->dt + n, false);
+    HIP_TRY(hipMemcpyAsync(T->lam, c->maxv[0], (size_t)c->K * 4 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     HIP_TRY(hipGetLastError());
     return DGLM_OK;
   }
@@ -1560,20 +1637,20 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
     T->nsteps = T->every = T->nck = 0;
     T->nkeep = -1;
     void *old[] = {T->keep, T->keep_lam, T->ckpt, T->ck_t, T->dt, T->seg, T->lam, T->kscr, T->fstar, T->clip,
-                   T->ck_step, T->scal2};
+                   T->ck_step, T->clk2};
     for (void *q : old)
       if (q) HIP_TRY(hipFree(q));
     T->keep = T->keep_lam = nullptr;
     T->keep_bytes = 0;
     T->ckpt = T->ck_t = T->dt = T->seg = T->lam = T->kscr = nullptr;
     T->fstar = T->clip = T->ck_step = nullptr;
-    T->scal2 = nullptr;
+    T->clk2 = nullptr;
     if ((rc = dev_alloc(&T->ckpt, nst * nck, "checkpoints")) || (rc = dev_alloc(&T->ck_t, (size_t)nck, "ckpt t")) ||
         (rc = dev_alloc(&T->ck_step, (size_t)nck, "ckpt step")) || (rc = dev_alloc(&T->dt, (size_t)nsteps, "dt")) ||
         (rc = dev_alloc(&T->fstar, (size_t)nsteps, "fstar")) || (rc = dev_alloc(&T->clip, (size_t)nsteps, "clip")) ||
         (rc = dev_alloc(&T->seg, nst * (5 * (size_t)every + 1), "segment states")) ||
         (rc = dev_alloc(&T->lam, (size_t)c->K * 4 * every, "segment wave speeds")) ||
-        (rc = dev_alloc(&T->kscr, nst, "k scratch")) || (rc = dev_alloc(&T->scal2, 1, "recompute scalars")))
+        (rc = dev_alloc(&T->kscr, nst, "k scratch")) || (rc = dev_alloc(&T->clk2, 2, "recompute clock")))
       return rc;
     T->nsteps = nsteps;
     T->every = every;
@@ -1616,13 +1693,18 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
     }
   }
   const int q0 = nck - T->nkeep;  // first kept segment
-  for (int n = 0; n < nsteps; n++) {
+  int ck = c->cur;  // clock slot of the step (it alternates also where the state buffer does not)
+  auto record_dt = [&](int n) {
+    hipLaunchKernelGGL(record_dt_kernel, dim3(1), dim3(1024), 0, c->stream, c->partial, c->partial_idx, c->nblk_ws,
+                       c->clk + ck, cfl_fac, c->p.tmax, T->dt + n, T->fstar + n, T->clip + n);
+  };
+  for (int n = 0; n < nsteps; n++, ck ^= 1) {
     const int q = n / every;
     if (n % every == 0) {
       HIP_TRY(hipMemcpyAsync(T->ckpt + nst * q, c->u[c->cur], nst * sizeof(double), hipMemcpyDeviceToDevice,
                              c->stream));
-      HIP_TRY(hipMemcpyAsync(T->ck_t + q, &c->scal->t_next, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      HIP_TRY(hipMemcpyAsync(T->ck_step + q, &c->scal->tstep, sizeof(int), hipMemcpyDeviceToDevice, c->stream));
+      HIP_TRY(hipMemcpyAsync(T->ck_t + q, &c->clk[ck].t, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+      HIP_TRY(hipMemcpyAsync(T->ck_step + q, &c->clk[ck].tstep, sizeof(int), hipMemcpyDeviceToDevice, c->stream));
     }
     if (q >= q0) {
       // a kept segment: the stages write straight into its tape slots (the
@@ -1632,24 +1714,25 @@ extern "C" int dglm_adjoint_record(dglm_ctx *c, int nsteps, int every) {
       double *lam = T->keep_lam + lam_n * (q - q0) + (size_t)c->K * 4 * (n - n0);
       if (n == n0)
         HIP_TRY(hipMemcpyAsync(base, c->u[c->cur], nst * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      ws(c, base, lam, c->partial, c->partial_idx);
-      hipLaunchKernelGGL(finalize_dt_kernel, dim3(1), dim3(1024), 0, c->stream, c->partial, c->partial_idx,
-                         c->nblk_ws, c->scal, cfl_fac, c->p.tmax, T->dt, T->fstar, T->clip, n);
-      for (int s = 0; s < 5; s++) st0(c, make_stage_args(c, base + nst * s, base + nst * (s + 1), c->k, lam, c->scal, s));
+      ws(c, base, lam, nullptr);
+      record_dt(n);
+      for (int s = 0; s < 5; s++)
+        st0(c, make_stage_args(c, base + nst * s, base + nst * (s + 1), c->k, lam, c->clk, ck, s));
       if (n == n1 - 1)  // the context's state continues from the segment's last stage
         HIP_TRY(hipMemcpyAsync(c->u[c->cur], base + nst * 5, nst * sizeof(double), hipMemcpyDeviceToDevice,
                                c->stream));
       continue;
     }
-    ws(c, c->u[c->cur], c->maxv, c->partial, c->partial_idx);
-    hipLaunchKernelGGL(finalize_dt_kernel, dim3(1), dim3(1024), 0, c->stream, c->partial, c->partial_idx,
-                       c->nblk_ws, c->scal, cfl_fac, c->p.tmax, T->dt, T->fstar, T->clip, n);
+    ws(c, c->u[c->cur], c->maxv[0], nullptr);
+    record_dt(n);
     for (int s = 0; s < 5; s++) {
-      StageArgs a = stage_args(c, s);
-      st0(c, a);
+      st0(c, make_stage_args(c, c->u[c->cur], c->u[c->cur ^ 1], c->k, c->maxv[0], c->clk, ck, s));
       c->cur ^= 1;
     }
   }
+  if (ck != c->cur)
+    hipLaunchKernelGGL(set_clock_kernel, dim3(1), dim3(MAXFS_SLOTS), 0, c->stream, c->clk + c->cur, c->clk + ck, 0, 0.0, 0);
+  stale_speeds(c);
   HIP_TRY(hipGetLastError());
   return DGLM_OK;
 }
@@ -1694,17 +1777,15 @@ extern "C" int dglm_adjoint_backward(dglm_ctx *c, const double *ubar_T, double *
     } else {
       // recompute the segment's stage states from its checkpoint
       HIP_TRY(hipMemcpyAsync(T->seg, T->ckpt + nst * q, nst * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      HIP_TRY(hipMemsetAsync(T->scal2, 0, sizeof(DevScalars), c->stream));
-      HIP_TRY(hipMemcpyAsync(&T->scal2->t_next, T->ck_t + q, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+      HIP_TRY(hipMemsetAsync(T->clk2, 0, 2 * sizeof(DevClock), c->stream));
+      HIP_TRY(hipMemcpyAsync(&T->clk2[0].t, T->ck_t + q, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
       for (int n = n0; n < n1; n++) {
+        const int ck = (n - n0) & 1;
         double *base = T->seg + nst * 5 * (size_t)(n - n0);
         double *lam = T->lam + (size_t)c->K * 4 * (n - n0);
-        ws(c, base, lam, c->partial, c->partial_idx);
-        hipLaunchKernelGGL(finalize_dt_kernel, dim3(1), dim3(1024), 0, c->stream, c->partial, c->partial_idx,
-                           c->nblk_ws, T->scal2, cfl_fac, c->p.tmax, (double *)nullptr, (int *)nullptr,
-                           (int *)nullptr, 0);
+        ws(c, base, lam, T->clk2 + ck);
         for (int s = 0; s < 5; s++)
-          st0(c, make_stage_args(c, base + nst * s, base + nst * (s + 1), T->kscr, lam, T->scal2, s));
+          st0(c, make_stage_args(c, base + nst * s, base + nst * (s + 1), T->kscr, lam, T->clk2, ck, s));
       }
     }
     // reverse sweep over the segment

@@ -206,8 +206,8 @@ int dglm_step(dglm_ctx *ctx, int nsteps, double *dt_hist);
  * tight serving loops, harnesses that forbid hipMalloc).  Advances nsteps like
  * dglm_step, with the same kernels and bitwise the same states and dt history
  * (dt_hist [nsteps], host, may be NULL), but calls no hipMalloc, hipFree or
- * allocating library routine: its device scratch -- the dt history and the
- * wave-speed block maxima -- lives in a fixed array of the library
+ * allocating library routine: its device scratch -- the dt history, and room for
+ * the wave-speed block maxima -- lives in a fixed array of the library
  * (DGLM_NOALLOC_SCRATCH_BYTES on every device it runs on, held until the
  * process ends), and the steps are launched one kernel at a time (no graph,
  * no timing events).  nsteps > DGLM_NOALLOC_MAX_STEPS, or a mesh with more
@@ -233,7 +233,8 @@ int dglm_sync(dglm_ctx *ctx);
 /* Per-kernel timing with HIP events on the context's stream (the reference
  * profiles with Nsight Compute, utils/src/python/gpu_profile.py:98-310).
  * Turning timing on resets the totals.  dglm_get_timing returns, for kernel
- * classes 0 = wave speed, 1 = dt finalize, 2 = fused stage, the summed
+ * classes 0 = wave speed (only where the step before did not leave it), 1 = dt
+ * (none: the stages form it themselves), 2 = fused stage, the summed
  * milliseconds and launch counts (synchronises the stream). */
 int dglm_set_timing(dglm_ctx *ctx, int on);
 

@@ -278,9 +278,11 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   __shared__ int s_fmx[16 * Nfp];
 
   double dt = 0.0;
-  const bool active = MODE == 1 || begin_stage(a, dt);
   const int batch = xcd_batch(order, nbatch);
-  if (batch < 0) return;
+  if (batch < 0) {
+    if (MODE == 0) begin_stage(a, dt);
+    return;
+  }
   const int e0 = batch * EB;
   const int K = a.K;
   const size_t KNp = (size_t)K * Np;
@@ -289,26 +291,18 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t n0 = (size_t)e0 * Np;
 
-  if (!active) {
-    // Past tmax: the stage is the identity on u (k untouched).
-    for (int v = 0; v < NV; v++)
-      for (int i = tid; i < ne * Np; i += NT) a.u_out[v * KNp + n0 + i] = a.u_in[v * KNp + n0 + i];
-    return;
-  }
-
-  // ---- 1. stage in.  Elements past the end of a short batch get a state at
-  // rest and no geometry; their columns are computed and not written ----
+  // ---- 1. stage in: every load before the first wait.  Elements past the end
+  // of a short batch get a state at rest and no geometry; their columns are
+  // computed and not written ----
   constexpr int RN = (EB * Np / VW + NT - 1) / NT;  // nodes (or pairs) per thread
   constexpr int RF = (EB * NFF + NT - 1) / NT;      // face nodes per thread
+  constexpr int RX = (16 * Nfp + NT - 1) / NT, RG = (EB * GEO_STRIDE + NT - 1) / NT;
   double lam_own = 0.0, lam_nbr = 0.0;
-  if (tid < 4 * EB) {
-    const int c = tid < 4 * ne ? a.conn[(size_t)e0 * 4 + tid] : 0;
-    s_conn[tid] = c;
-    s_dm[tid] = a.dmap && tid < 4 * ne ? a.dmap[(size_t)e0 * 4 + tid] : -1;
-    if (tid < 4 * ne) {
-      lam_own = a.maxv[(size_t)e0 * 4 + tid];
-      lam_nbr = a.maxv[(size_t)conn_nbr(c) * 4 + conn_face(c)];
-    }
+  int cw = 0, dm = -1;
+  if (tid < 4 * ne) {
+    cw = a.conn[(size_t)e0 * 4 + tid];
+    if (a.dmap) dm = a.dmap[(size_t)e0 * 4 + tid];
+    lam_own = a.maxv[(size_t)e0 * 4 + tid];
   }
   vec un[RN][NV], vl[EUL ? 1 : RN][3];
 #pragma unroll
@@ -328,8 +322,30 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
       }
     }
   }
-  for (int i = tid; i < 16 * Nfp; i += NT) s_fmx[i] = a.fmx[i];
-  for (int i = tid; i < EB * GEO_STRIDE; i += NT) s_geo[i] = i < ne * GEO_STRIDE ? a.geo[(size_t)e0 * GEO_STRIDE + i] : 0.0;
+  int fx[RX];
+  double gx[RG];
+#pragma unroll
+  for (int r = 0; r < RX; r++) fx[r] = tid + NT * r < 16 * Nfp ? a.fmx[tid + NT * r] : 0;
+#pragma unroll
+  for (int r = 0; r < RG; r++)
+    gx[r] = tid + NT * r < ne * GEO_STRIDE ? a.geo[(size_t)e0 * GEO_STRIDE + tid + NT * r] : 0.0;
+  if (MODE == 0 && !begin_stage(a, dt)) {
+    // Past tmax: the stage is the identity on u (k untouched).
+    for (int v = 0; v < NV; v++)
+      for (int i = tid; i < ne * Np; i += NT) a.u_out[v * KNp + n0 + i] = a.u_in[v * KNp + n0 + i];
+    return;
+  }
+  if (tid < 4 * EB) {
+    s_conn[tid] = cw;
+    s_dm[tid] = dm;
+    if (tid < 4 * ne) lam_nbr = a.maxv[(size_t)conn_nbr(cw) * 4 + conn_face(cw)];
+  }
+#pragma unroll
+  for (int r = 0; r < RX; r++)
+    if (tid + NT * r < 16 * Nfp) s_fmx[tid + NT * r] = fx[r];
+#pragma unroll
+  for (int r = 0; r < RG; r++)
+    if (tid + NT * r < EB * GEO_STRIDE) s_geo[tid + NT * r] = gx[r];
   if constexpr (Np % 4 != 0) {  // nodes Np..4G-1
     for (int i = tid; i < EB * (4 * G - Np); i += NT) {
       const int o = i / (4 * G - Np) * NS + Np + i % (4 * G - Np);
@@ -369,6 +385,11 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
       }
     }
   }
+  // Pressure and contravariant velocity (fluxes) of this thread's nodes.  In a
+  // closure because the compiler then keeps its index arithmetic out of the
+  // phases after it: 158 VGPRs for N = 3 [6,1] and 85 for N = 5 [3,4], written
+  // inline 160 and 93 (5 to 6% slower stages).
+  auto primitives = [&]() {
 #pragma unroll
   for (int r = 0; r < RN; r++) {
     const int i = (tid + NT * r) * VW;
@@ -401,6 +422,8 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   }
   if (tid < 4 * EB) s_tau[tid] = 0.25 * (lam_own + lam_nbr) * a.tau_scale;
   lds_barrier();
+  };
+  primitives();
 
   const int kk = lane >> 4, cl = lane & 15;
   constexpr int RO = (NC * Np / VW + NT - 1) / NT;  // values (or pairs) of the update per thread
@@ -418,6 +441,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
     constexpr int T = role.nt, XT = role.xt >= 0 ? 1 : 0, Q = role.nq, NA = role.na();
     constexpr int T1 = T > 0 ? T : 1, Q1 = Q > 0 ? Q : 1;
     const double *ap = afrag + stream;
+    ColA<NA> A[2];
     f64x4 acc[T1][CT], acx = {0.0, 0.0, 0.0, 0.0};
     double acq[Q1][CT];
 #pragma unroll
@@ -437,7 +461,6 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
       cv[t] = c < NC ? c / EB : 0;
       ce[t] = c < NC ? c - cv[t] * EB : 0;
     }
-    ColA<NA> A[2];
     auto contract = [&](const ColA<NA> &Ad, const double (&Bd)[3][CT], int n) {
 #pragma unroll
       for (int d = 0; d < 3; d++) {
@@ -685,22 +708,32 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   }
 }
 
-// Elements per workgroup and waves: a large and a small configuration of each
-// order.  Measured in us per stage (uniform vortex meshes, Rusanov flux;
-// [EB, waves]):
-//   Euler, K =   1296        6000        13182        24576       82944
-//   N = 2   [3,2] 7.0 [9,2] 7.9   10.1  10.9   18.2  15.4   31.1  26.6
-//   N = 3   [3,2] 7.8 [9,2] 10.5  12.4  15.3   24.1  22.9   39.4  39.5
-//   N = 4   [3,4] 9.7 [9,2] 15.9  23.3  27.0   43.9  50.8   77.7  78.1
-//   N = 5   [3,4] 12.1 [12,4] 18.6  35.9  35.4  72.2  78.2  142  129    488  431
-//   N = 6   [6,4] 20.3 [9,4] 23.5  58.6  62.4   128  126    228  225    714  698
-//   N = 7   [6,4] 29.6 [3,4] 29.4  99.8 107     220  229    399  436
+// Elements per workgroup and waves: a small-mesh and a large-mesh configuration
+// of each order.  Measured in us per stage, launch included (uniform vortex
+// meshes, Rusanov flux; [EB, waves]):
+//   Euler, K =            1296   6000   10368  13182  20250  82944
+//   N = 1   [6,2]          7.2    8.2    9.7   10.5   13.5   33.8
+//           [16,1]         8.4    9.0    9.6   10.4   12.1   25.5
+//   N = 2   [3,2]          8.1   11.3   15.5   18.0   23.9   78.7
+//           [6,1]          9.3   11.1   14.1   16.5   20.8   56.2
+//   N = 3   [3,2]          8.9   13.9   20.3   22.7   31.4    105
+//           [6,1]         11.5   14.5   19.6   23.3   33.7   93.9
+//   N = 4   [3,4]         11.9   24.8   36.1   45.1   66.2    206
+//           [6,2]         14.3   23.1   39.0   45.0   61.7    207
+//   N = 5   [3,4]         14.4   37.1   56.4   69.3    103    401
+//           [6,2]         19.8   35.2   62.2   69.7   98.7    359
+//   N = 6   [6,4]         21.5   59.7   93.7    116    168    617
+//           [9,4]         26.2   62.6    101    118    166    617
+//   advection N = 5 [16,8] 10.5  14.5   21.5          35.4    117
+//                   [16,4] 10.9  14.9   20.5          32.7    106
 // Few elements per workgroup while the mesh does not fill the GPU (a stage is
-// then one pass of the chain load, gather, flux, contraction, store), many once
-// it does (each operator load then serves more columns); above N = 7 the LDS
-// holds three elements beside a second workgroup.  For advection a column
-// tile is 16 elements, and 32 were slower (N = 4: 84 against 63 us at K =
-// 82,944; N = 5: 73 against 67 at 48,000).
+// then one pass of the chain load, gather, flux, contraction, store), many to a
+// wave once it does: each operator load then serves more columns, and fewer
+// waves meet at a barrier (Euler N = 3, K = 82,944: [9,2] 107, [6,1] 99; N = 5:
+// [12,4] 371, [6,2] 356, in one run).  Nine or more elements in fewer waves
+// leave two waves a SIMD (N = 5 [9,2] 444).  Above N = 7 the LDS holds three
+// elements beside a second workgroup.  For advection a column tile is 16
+// elements, and 32 were slower (N = 4: 84 against 63 us at K = 82,944).
 struct ColConfig {
   int eb, nw;
 };
@@ -708,14 +741,13 @@ constexpr ColConfig cols_config(int N, int phys, bool small) {
   if (phys == PHYS_ADV) return {16, N <= 2 ? N : (N <= 4 || (N <= 6 && !small) ? 4 : 8)};
   switch (N) {
     case 1:
-      return small ? ColConfig{6, 2} : ColConfig{16, 2};
+      return small ? ColConfig{6, 2} : ColConfig{16, 1};
     case 2:
     case 3:
-      return small ? ColConfig{3, 2} : ColConfig{9, 2};
+      return small ? ColConfig{3, 2} : ColConfig{6, 1};
     case 4:
-      return small ? ColConfig{3, 4} : ColConfig{9, 2};
     case 5:
-      return small ? ColConfig{3, 4} : ColConfig{12, 4};
+      return small ? ColConfig{3, 4} : ColConfig{6, 2};
     case 6:
       return small ? ColConfig{6, 4} : ColConfig{9, 4};
     case 7:
@@ -724,11 +756,11 @@ constexpr ColConfig cols_config(int N, int phys, bool small) {
       return {3, 4};
   }
 }
-// Whether a mesh of K elements takes the small configuration: about where the
-// columns above cross (in small batches: eight a CU; at N = 4 thirty-two).
+// Whether a mesh of K elements takes the small-mesh configuration: about where
+// the lines above cross, in small batches.
 constexpr bool cols_small(int N, int phys, int K) {
   const int nb = (K + cols_config(N, phys, true).eb - 1) / cols_config(N, phys, true).eb;
-  return nb <= (phys == PHYS_EULER && N == 4 ? 8192 : 2048);
+  return nb <= (phys == PHYS_ADV ? 512 : N >= 3 && N <= 5 ? 6144 : 2048);
 }
 
 template <int N, int PHYS, bool SMALL>

@@ -809,7 +809,9 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   std::vector<int> ws_order, cols_order;
   if (!centroid.empty()) {
     if (!afr_ws.empty() || !mx_tab.empty()) ws_order = batch_order(centroid, 16);
-    if (!cfr.empty()) cols_order = batch_order(centroid, cops.eb);
+    // (a small mesh is in the L2 whatever the order, and its stages are chains of
+    // loads, of which the table would be one more)
+    if (!cfr.empty() && (K + cops.eb - 1) / cops.eb > 2048) cols_order = batch_order(centroid, cops.eb);
   }
 
   dglm_ctx *c = new dglm_ctx();

@@ -54,7 +54,8 @@ def _check(pb, physics, flux, u, kernel, steps=2):
 
 @pytest.mark.parametrize("flux", ["lm", "rusanov"])
 @pytest.mark.parametrize("physics,N,nhex", [("euler", 1, 13), ("euler", 2, 11), ("euler", 3, 11), ("euler", 4, 17),
-                                            ("euler", 5, 11), ("euler", 6, 13), ("euler", 7, 5), ("euler", 10, 3),
+                                            ("euler", 5, 11), ("euler", 6, 13), ("euler", 7, 5), ("euler", 10, 3), ("euler", 3, 15),
+                                            ("euler", 5, 15),
                                             ("advection", 1, 13), ("advection", 2, 13), ("advection", 5, 18),
                                             ("advection", 6, 18), ("advection", 8, 5)])
 def test_large_meshes(gpu, physics, N, nhex, flux):

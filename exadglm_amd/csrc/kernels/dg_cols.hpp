@@ -194,6 +194,16 @@ __device__ inline void cols_surface_flux5(const double uM[5], const double uP[5]
 // (nothing in a launch reads global memory that the launch writes).
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Value at a byte offset from a wave-uniform address.
+template <class V>
+__device__ inline V &at_offset(double *base, unsigned off) {
+  return *reinterpret_cast<V *>(reinterpret_cast<char *>(base) + off);
+}
+template <class V>
+__device__ inline V at_offset(const double *base, unsigned off) {
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + off);
+}
+
 // A lane's operator values of one block.
 template <int NA>
 struct ColA {
@@ -273,7 +283,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   __shared__ __align__(16) double s_x[S::X];
   __shared__ double s_geo[EB * GEO_STRIDE];
   __shared__ double s_tau[EB * 4];
-  __shared__ int s_conn[EB * 4];
+  __shared__ int2 s_conn[EB * 4];  // exterior element, row of its trace in s_fmx
   __shared__ int s_dm[EB * 4];
   __shared__ int s_fmx[16 * Nfp];
 
@@ -291,8 +301,8 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t n0 = (size_t)e0 * Np;
 
-  // ---- 1. stage in: every load before the first wait.  Elements past the end
-  // of a short batch get a state at rest and no geometry; their columns are
+  // ---- 1. stage in: every load before the first wait.  Threads past the end of
+  // a short batch repeat its last node; the columns of elements past it are
   // computed and not written ----
   constexpr int RN = (EB * Np / VW + NT - 1) / NT;  // nodes (or pairs) per thread
   constexpr int RF = (EB * NFF + NT - 1) / NT;      // face nodes per thread
@@ -304,21 +314,18 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
     if (a.dmap) dm = a.dmap[(size_t)e0 * 4 + tid];
     lam_own = a.maxv[(size_t)e0 * 4 + tid];
   }
+  // waves that the last round leaves without a node skip it
+  auto some = [&](int r) { return (NT * (r + 1) - 64) * VW < EB * Np || (64 * w + NT * r) * VW < EB * Np; };
   vec un[RN][NV], vl[EUL ? 1 : RN][3];
 #pragma unroll
   for (int r = 0; r < RN; r++) {
-    const int i = (tid + NT * r) * VW;
-    const bool live = i < ne * Np;
+    const unsigned off = 8u * min((tid + NT * r) * VW, ne * Np - VW);
+    if (some(r)) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      un[r][v] = vec(EUL && v == 0 ? 1.0 : 0.0);
-      if (live) un[r][v] = *reinterpret_cast<const vec *>(a.u_in + v * KNp + n0 + i);
-    }
-    if constexpr (!EUL) {
+      for (int v = 0; v < NV; v++) un[r][v] = at_offset<vec>(a.u_in + (v * KNp + n0), off);
+      if constexpr (!EUL) {
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        vl[r][d] = vec(0.0);
-        if (live) vl[r][d] = *reinterpret_cast<const vec *>(a.vel + d * KNp + n0 + i);
+        for (int d = 0; d < 3; d++) vl[r][d] = at_offset<vec>(a.vel + (d * KNp + n0), off);
       }
     }
   }
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
     return;
   }
   if (tid < 4 * EB) {
-    s_conn[tid] = cw;
+    s_conn[tid] = make_int2(conn_nbr(cw), (conn_face(cw) * 4 + conn_code(cw)) * Nfp);
     s_dm[tid] = dm;
     if (tid < 4 * ne) lam_nbr = a.maxv[(size_t)conn_nbr(cw) * 4 + conn_face(cw)];
   }
@@ -364,14 +371,15 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   for (int r = 0; r < RF; r++) {
     const int idx = min(tid + NT * r, EB * NFF - 1), e = idx / NFF, m = idx - e * NFF;
     const int f = m / Nfp, j = m - f * Nfp;
-    const int c = s_conn[e * 4 + f];
-    const size_t pi = (size_t)conn_nbr(c) * Np + s_fmx[(conn_face(c) * 4 + conn_code(c)) * Nfp + j];
+    const int2 c = s_conn[e * 4 + f];
+    const int n = s_fmx[c.y + j];
+    const size_t pi = (size_t)c.x * Np + n;
 #pragma unroll
     for (int v = 0; v < NV; v++) uP[r][v] = a.u_in[v * KNp + pi];
     if constexpr (!EUL) {
-      const size_t mi = e < ne ? n0 + e * Np + s_fmx[(f * 4 + 3) * Nfp + j] : 0;
+      const unsigned o = e < ne ? 8u * (e * Np + s_fmx[(f * 4 + 3) * Nfp + j]) : 0;
 #pragma unroll
-      for (int d = 0; d < 3; d++) vf[r][d] = a.vel[d * KNp + mi];
+      for (int d = 0; d < 3; d++) vf[r][d] = at_offset<double>(a.vel + (d * KNp + n0), o);
     }
   }
   if (a.dmap) {  // Dirichlet faces: the prescribed state instead
@@ -426,14 +434,13 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
   primitives();
 
   const int kk = lane >> 4, cl = lane & 15;
-  constexpr int RO = (NC * Np / VW + NT - 1) / NT;  // values (or pairs) of the update per thread
-  // value i of the update: variable, offset in its batch of nodes, LDS place
-  auto place = [&](int i, int &v, int &n, int &o) {
-    v = i / (EB * Np);
-    n = i - v * (EB * Np);
-    const int e = n / Np;
-    o = (v * EB + e) * NS + n - e * Np;
-  };
+  // Update: thread's nodes as in phase 1, all variables; where half the waves or
+  // more would be left without a node, groups of UW waves take the variables in
+  // turn (a wave has one variable at a time, so its rows' addresses are scalar)
+  constexpr int UW = (EB * Np / VW + 63) / 64, UG = NW / UW > 1 ? NW / UW : 1;
+  constexpr int RU = UG > 1 ? 1 : RN, RV = (NV + UG - 1) / UG;
+  const int ug = UG > 1 ? w / UW : 0, ut = UG > 1 ? tid - ug * 64 * UW : tid;
+  auto mine = [&](int r, int q) { return UG > 1 ? ug < UG && q * UG + ug < NV : some(r); };
 
   // phases 2..4 of a wave
   auto body = [&](auto role_, size_t stream, int tile0, int xt, int c0, int q0) {
@@ -579,16 +586,16 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
     lds_barrier();
 
     // ---- 4. surface k-steps; the LSRK registers arrive meanwhile ----
-    vec kr[RO];
+    vec kr[RU][RV];
     if (MODE == 0) {
 #pragma unroll
-      for (int r = 0; r < RO; r++) {
-        const int i = (tid + NT * r) * VW;
-        int v, n, o;
-        place(min(i, NC * Np - VW), v, n, o);
-        kr[r] = vec(0.0);
-        if (a.rka != 0.0 && n < ne * Np) kr[r] = *reinterpret_cast<const vec *>(a.k + v * KNp + n0 + n);
-      }
+      for (int r = 0; r < RU; r++)
+#pragma unroll
+        for (int q = 0; q < RV; q++) {
+          kr[r][q] = vec(0.0);
+          if (a.rka != 0.0 && mine(r, q))
+            kr[r][q] = at_offset<vec>(a.k + ((q * UG + ug) * KNp + n0), 8u * min((ut + NT * r) * VW, ne * Np - VW));
+        }
     }
     if constexpr (NA > 0) {
       constexpr int SB = S::SB;
@@ -644,21 +651,26 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
 
     // ---- LSRK update, in memory order ----
 #pragma unroll
-    for (int r = 0; r < RO; r++) {
-      const int i = (tid + NT * r) * VW;
-      int v, n, o;
-      place(min(i, NC * Np - VW), v, n, o);
-      if (i < NC * Np && n < ne * Np) {
-        const size_t gi = v * KNp + n0 + n;
-        const vec rhs = *reinterpret_cast<const vec *>(&s_x[o]);
-        if (MODE == 1) {
-          *reinterpret_cast<vec *>(a.rhs + gi) = rhs;
-        } else {
-          const vec kn = a.rka * kr[r] + dt * rhs;
-          if (a.k_out) *reinterpret_cast<vec *>(a.k + gi) = kn;
-          const vec u1 = *reinterpret_cast<const vec *>(&s_u[o]) + a.rkb * kn;
-          *reinterpret_cast<vec *>(a.u_out + gi) = u1;
-          if (EUL && a.lam_out) *reinterpret_cast<vec *>(&s_u[o]) = u1;
+    for (int r = 0; r < RU; r++) {
+      const int i = (ut + NT * r) * VW;
+      if (i < ne * Np) {
+        const int e = i / Np, o = e * NS + i - e * Np;
+#pragma unroll
+        for (int q = 0; q < RV; q++) {
+          if (UG > 1 && !mine(r, q)) continue;
+          const int v = q * UG + ug;
+          const size_t row = v * KNp + n0;
+          const vec rhs = *reinterpret_cast<const vec *>(&s_x[v * EB * NS + o]);
+          if (MODE == 1) {
+            at_offset<vec>(a.rhs + row, 8u * i) = rhs;
+          } else {
+            const vec kn = a.rka * kr[r][q] + dt * rhs;
+            if (a.k_out) at_offset<vec>(a.k + row, 8u * i) = kn;
+            vec &u = *reinterpret_cast<vec *>(&s_u[v * EB * NS + o]);
+            const vec u1 = u + a.rkb * kn;
+            at_offset<vec>(a.u_out + row, 8u * i) = u1;
+            if (EUL && a.lam_out) u = u1;
+          }
         }
       }
     }

@@ -109,15 +109,15 @@ def profiled_traffic(ksym, args):
     summary of this workload (FETCH_SIZE x 2 + WRITE_SIZE x 1 KiB per dispatch,
     factors from a plain copy of known size), when the summary covers this
     kernel and configuration; (None, None) otherwise."""
-    path = os.path.join("profiles", f"stage_ws_kernel_euler_N{args.order}_K{6 * args.nhex ** 3}.txt")
-    if ksym != f"stage_ws_kernel<{args.order}, 0, false>" or args.precision != "fp64" or \
+    path = os.path.join("profiles", f"stage_wave_kernel_euler_N{args.order}_K{6 * args.nhex ** 3}.txt")
+    if not ksym.startswith("stage_wave_kernel<") or args.precision != "fp64" or \
             not os.path.exists(os.path.join(ROOT, path)):
         return None, None
     in_table = False  # the memory-counter table: ... disp, FETCH KiB, WRITE KiB, HBM MB
     for line in open(os.path.join(ROOT, path)):
         if "FETCH KiB" in line and "WRITE KiB" in line:
             in_table = True
-        elif in_table and line.startswith(f"void dglm::stage_ws_kernel<{args.order}, 0, false>"):
+        elif in_table and line.startswith(f"void dglm::{ksym}"):
             f = line.split()
             try:
                 fetch, write = float(f[-3]), float(f[-2])
@@ -355,7 +355,7 @@ def main():
         roof = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS}
     else:
         roof = {"bound": "mfma", "achieved": tfl, "peak": pk, "unit": "TFLOP/s", "frac": tfl / pk}
-    ksym = f"stage_ws_kernel<{args.order}, 0, false>" if kernel_name == "mfma_ws" else \
+    ksym = f"stage_wave_kernel<{args.order}, {6 if args.order == 3 else 3}, 8, 0>" if kernel_name == "mfma_ws" else \
         f"stage_{kernel_name}_kernel<{args.order}, EULER, 0>"
     roof["traffic"], roof["traffic_source"] = profiled_traffic(ksym, args)
     roof["kernel"] = ksym
@@ -416,7 +416,7 @@ def main():
             grads = {}
             # the mixed-precision configuration's FP32-MFMA forward is the fused
             # mixed kernel, selected explicitly: an FP32 request at N = 4 (AUTO)
-            # runs the FP64 warp-specialised kernel, which is faster there
+            # runs the persistent FP64 kernel, which is faster there
             for prec in ("fp64", "fp32"):
                 res = adjoint_leg(prec, stage_kernel="mfma_mx" if prec == "fp32" else None)
                 grads[prec] = res.pop("grad")

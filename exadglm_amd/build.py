@@ -19,7 +19,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 HOST_SRCS = ["host/refelem.cpp", "host/mesh.cpp", "host/datain.cpp"]
-HIP_SRCS = ["solver.hip", "ws_dirichlet.hip", "cols_euler_low.hip", "cols_euler_high.hip", "cols_advection.hip",
+HIP_SRCS = ["solver.hip", "wave_euler.hip", "cols_euler_low.hip", "cols_euler_high.hip", "cols_advection.hip",
             "adjoint_advection.hip", "adjoint_euler.hip"]
 
 HIP_FLAGS = [

@@ -14,10 +14,8 @@ struct Ord {
   static constexpr int KD = 3 * Np + NFF;  // stacked contraction length [WDr|WDs|WDt|LIFT]
 };
 
-// Reciprocal and square root for dependency chains that bound a kernel (the
-// fused mixed-precision kernel's surface and volume passes; in the adjoint's
-// pass A and the FP64 warp-specialised kernel they were measured no faster): the
-// hardware estimates v_rcp_f64 and v_rsq_f64 refined by Newton steps (two
+// Reciprocal and square root of the stage kernels (the adjoint's pass A, where
+// they were measured no faster, divides): the hardware estimates v_rcp_f64 and v_rsq_f64 refined by Newton steps (two
 // r += r (1 - x r); for the root a coupled step on g = x y, h = y / 2 and a
 // correction g += h (x - g^2)), within an ulp of the IEEE results and equal
 // to them on every one of 4M sampled densities in [1e-3, 1e3] and squared

@@ -4,7 +4,7 @@
 //
 // Math follows the reference CPU path:
 //   calc_maxv   dim3/src/cpp/euler_dglm.cpp:6-50,   advec_dglm.cpp:6-35
-//               (its kernel, wavespeed_lds_kernel, is in dg_ws.hpp)
+//               (its kernel, wavespeed_lds_kernel, is in dg_wavespeed.hpp)
 //   calc_dt     euler_dglm.cpp:53-69 (its kernel is in dg_step.hpp)
 //   update_tau  euler_dglm.cpp:72-84
 //   update_ub + calc_fluxLM  euler_dglm.cpp:87-183, advec_dglm.cpp:69-133

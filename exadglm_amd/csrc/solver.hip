@@ -24,20 +24,14 @@
 #include "host/mesh.h"
 #include "host/refelem.h"
 #include "kernels/cols_ops.h"
+#include "kernels/wave_ops.h"
 #include "kernels/dg_fp64.hpp"
 #include "kernels/dg_step.hpp"
 #include "kernels/dg_mfma.hpp"
-#include "kernels/dg_ws.hpp"
+#include "kernels/dg_wavespeed.hpp"
 #include "kernels/dg_mx.hpp"
 #include "kernels/adjoint_ops.h"
 #include "kernels/dg_adjoint.hpp"
-
-namespace dglm {
-// ws_dirichlet.hip: the warp-specialised stage kernel on meshes with Dirichlet
-// faces (false: not built for this order).
-bool launch_ws_dirichlet(int N, int mode, int grid, hipStream_t stream, const StageArgs &a, const double *afrag,
-                         const double *arem, const int *order, int nbatch, int groups);
-}  // namespace dglm
 
 #define DGLM_NTIMERS 3  // wave speed, (none), stage
 
@@ -105,12 +99,13 @@ struct dglm_ctx {
   int *cols_order = nullptr;      // its batch visiting order (null: mesh order)
   double *rowsum = nullptr;       // FP64 affine-offset tables of the mixed-precision contraction
   int mfma_grid = 0;              // persistent grid size (0 = not yet sized)
-  double *afrag_ws = nullptr;     // operator rows in the warp-specialised kernel's k order
-  double *arem_ws = nullptr;      // rows left to the VALU by that kernel
-  int *ws_order = nullptr;        // its batch visiting order (null: mesh order)
+  WaveOps wave;                   // the persistent one-wave-per-batch kernel's entry points (none: eb 0)
+  double *op_wave = nullptr;      // its operator (null: not for this solver)
+  int *wave_order = nullptr;      // its batch visiting order (null: mesh order)
+  int cus = 0;                    // compute units of the device
   unsigned char *mx_tab = nullptr;  // tables of the mixed-precision Euler kernel (null: not built)
+  int *mx_order = nullptr;           // its batch visiting order (null: mesh order)
   int mx_grid = 0, mx_groups = 1;    // its persistent grid and XCD groups
-  int ws_grid = 0, ws_groups = 1;  // its persistent grid and XCD groups
   struct dglm_adj_tape *tape = nullptr;  // adjoint buffers and recorded trajectory
   bool use_graph = true;                 // replay two-step hipGraphs in dglm_step
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // keyed by the state buffer the step starts from
@@ -292,67 +287,36 @@ void launch_wavespeed(dglm_ctx *c, const double *u, double *maxv, DevClock *clk)
 // packed-column kernel is the only FP64 kernel and goes by the name SIMPLE).
 inline bool mfma_available(int N) { return N >= 1 && N <= 6; }
 
-// The warp-specialised kernel pipelines over the 16-element batches of a
-// persistent workgroup; below this many elements (five batches for each of 256
-// CUs) the packed-column kernel is faster at N = 4 (K = 11,520: 37 against 44
-// us per stage; 16,464: 54 and 60; 24,576: 77 and 74; 48,000: 140 and 127).
-constexpr int WS_MIN_ELEMS = 16 * 5 * 256;
-
-// True when the warp-specialised kernel exists for this order.
-inline bool ws_built(int N) {
-  switch (N) {
-    case 3:
-      return ws_available<3>();
-    case 4:
-      return ws_available<4>();
-    default:
-      return false;
-  }
+// Whether the persistent kernel (one wave per batch, dg_wave.hpp) is the faster
+// one on this FP64 mesh: its waves take batches in rounds, so the last round
+// should leave few of them idle, and below one round of order 4 the packed-column
+// kernel also leaves the next step's wave speeds.  Measured (us per stage, LM
+// flux, packed columns / persistent):
+//   N = 3 (12,288 elements a round)   K = 6000 13.5/16.6, 10,368 19.5/18.2, 13,182
+//     22.1/26.7, 20,250 31.2/27.8, 48,000 54.7/49.8, 196,608 223/185
+//   N = 4 (6144 a round)   K = 7986 29.5/31.8, 10,368 35.8/32.9, 13,182 42.8/42.5,
+//     20,250 58.4/53.6, 48,000 116/101, 196,608 464/362
+bool wave_fills(const dglm_ctx *c) {
+  const long per_round = (long)(c->cus / 8 * 8) * c->wave.nw * c->wave.eb;
+  const long rounds = (c->K + per_round - 1) / per_round;
+  return c->K > 6144 && 5L * c->K >= 4 * rounds * per_round;
 }
 
 // The stage kernel that runs: the request where it exists, else the best
 // available.  FP64: the packed-column kernel (MFMA; SIMPLE above N = 6), but at
-// N = 4 on large Euler meshes the warp-specialised one (at N = 3 the packed
-// columns are faster at every size: K = 1296: 7.8 against 14.6 us per stage,
-// 24,576: 39 and 48, 384,000: 571 and 603).  DGLM_FP32: the warp-specialised
-// kernel at N = 3, 4, else the fused mixed-precision kernel (Euler), else the
-// generic MFMA kernel.
+// N = 3, 4 on Euler meshes that fill it the persistent one (MFMA_WS).
+// DGLM_FP32: the persistent kernel at N = 3, 4, else the fused mixed-precision
+// kernel (Euler), else the generic MFMA kernel.
 int stage_kind(const dglm_ctx *c) {
-  const bool ws = c->afrag_ws != nullptr, fp64 = c->p.precision == DGLM_FP64;
+  const bool ws = c->op_wave != nullptr, fp64 = c->p.precision == DGLM_FP64;
   const bool mf = mfma_available(c->p.N) && (fp64 || c->afrag != nullptr);
   if (c->variant == DGLM_STAGE_SIMPLE && fp64) return DGLM_STAGE_SIMPLE;
   if (c->variant == DGLM_STAGE_MFMA && mf) return DGLM_STAGE_MFMA;
   if (c->variant == DGLM_STAGE_MFMA_MX && c->mx_tab) return DGLM_STAGE_MFMA_MX;
-  if (ws && (c->variant == DGLM_STAGE_MFMA_WS || !fp64 || (c->p.N == 4 && c->K >= WS_MIN_ELEMS)))
+  if (ws && (c->variant == DGLM_STAGE_MFMA_WS || !fp64 || wave_fills(c)))
     return DGLM_STAGE_MFMA_WS;
   if (c->mx_tab) return DGLM_STAGE_MFMA_MX;
   return mf ? DGLM_STAGE_MFMA : DGLM_STAGE_SIMPLE;
-}
-
-template <int N, int MODE>
-void launch_ws(dglm_ctx *c, const StageArgs &a) {
-  if constexpr (ws_available<N>()) {
-    using S = WsShape<N>;
-    const int nbatch = (c->K + S::EB - 1) / S::EB;
-    if (c->ws_grid == 0) {
-      int dev = 0, cus = 0, occ = 0;
-      hipGetDevice(&dev);
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_ws_kernel<N, 0, false>, S::NT, 0);
-      c->ws_grid = (cus > 0 ? cus : 256) * (occ > 0 ? occ : 1);
-      c->ws_groups = c->ws_grid % 8 == 0 ? 8 : 1;
-    }
-    int grid = c->ws_grid, groups = c->ws_groups;
-    if (nbatch < grid) {
-      grid = nbatch;
-      groups = 1;
-    }
-    if (a.dmap)
-      launch_ws_dirichlet(N, MODE, grid, c->stream, a, c->afrag_ws, c->arem_ws, c->ws_order, nbatch, groups);
-    else
-      hipLaunchKernelGGL((stage_ws_kernel<N, MODE, false>), dim3(grid), dim3(S::NT), 0, c->stream, a, c->afrag_ws,
-                         c->arem_ws, c->ws_order, nbatch, groups);
-  }
 }
 
 template <int N, int MODE>
@@ -373,7 +337,7 @@ void launch_mx(dglm_ctx *c, const StageArgs &a) {
       grid = nbatch;
       groups = 1;
     }
-    hipLaunchKernelGGL((stage_mx_kernel<N, MODE>), dim3(grid), dim3(S::NT), 0, c->stream, a, c->mx_tab, c->ws_order,
+    hipLaunchKernelGGL((stage_mx_kernel<N, MODE>), dim3(grid), dim3(S::NT), 0, c->stream, a, c->mx_tab, c->mx_order,
                        nbatch, groups);
   }
 }
@@ -398,7 +362,7 @@ template <int N, int PHYS, int MODE>
 void launch_stage(dglm_ctx *c, const StageArgs &a) {
   const int kind = stage_kind(c);
   if (PHYS == PHYS_EULER && kind == DGLM_STAGE_MFMA_WS) {
-    launch_ws<N, MODE>(c, a);
+    c->wave.launch(MODE, c->cus, c->stream, a, c->op_wave, c->wave_order);
     return;
   }
   if (PHYS == PHYS_EULER && kind == DGLM_STAGE_MFMA_MX) {
@@ -510,8 +474,8 @@ void free_ctx(dglm_ctx *c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   void *ptrs[] = {c->u[0], c->u[1], c->k, c->rhs, c->vel, c->geo, c->op, c->maxv[0],
                   c->maxv[1] != c->maxv[0] ? c->maxv[1] : nullptr, c->partial, c->dt_hist,
-                  c->conn, c->fmx, c->clk, c->afrag, c->rowsum, c->partial_idx, c->afrag_ws, c->arem_ws,
-                  c->ws_order, c->dmap, c->gbnd, c->mx_tab, c->afrag_cols, c->cols_order};
+                  c->conn, c->fmx, c->clk, c->afrag, c->rowsum, c->partial_idx, c->op_wave, c->wave_order,
+                  c->mx_order, c->dmap, c->gbnd, c->mx_tab, c->afrag_cols, c->cols_order};
   for (void *q : ptrs)
     if (q) hipFree(q);
   if (c->h_rep) hipHostFree(c->h_rep);
@@ -760,25 +724,17 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   }
   const size_t afrag_bytes = afr32.size() * sizeof(float) + afrbf.size() * sizeof(s16x4);
   const void *afrag_src = !afr32.empty() ? (const void *)afr32.data() : (const void *)afrbf.data();
-  // Operator rows for the warp-specialised FP64 Euler kernel, which also runs
-  // DGLM_FP32 at the orders it is built for (N = 3, 4): there its FP64
+  // Operator of the persistent one-wave-per-batch FP64 Euler kernel, which also
+  // runs DGLM_FP32 at the orders it is built for (N = 3, 4): there its FP64
   // contraction outruns the fused mixed-precision kernel, whose least-squares
   // fits cost more FP64 work than the FP32 MFMA saves when the stage is bound
   // by the FP64 flux arithmetic, and it is exact where FP32 promises 1e-8.
-  std::vector<double> afr_ws, arem_ws;
-  // (its gathers index one variable's nodes with 32-bit offsets)
-  if (p->physics == DGLM_EULER && (p->precision == DGLM_FP64 || p->precision == DGLM_FP32) && ws_built(p->N) &&
-      (long long)K * Np < (1LL << 31)) {
-    if (p->N == 3) {
-      afr_ws.resize((size_t)WsShape<3>::RTF * WsShape<3>::KS * 64);
-      arem_ws.resize((size_t)WsShape<3>::REM * WsShape<3>::KDP);
-      ws_arrange<3>(op.data(), afr_ws.data(), arem_ws.data());
-    } else {
-      afr_ws.resize((size_t)WsShape<4>::RTF * WsShape<4>::KS * 64);
-      arem_ws.resize((size_t)WsShape<4>::REM * WsShape<4>::KDP);
-      ws_arrange<4>(op.data(), afr_ws.data(), arem_ws.data());
-    }
-  }
+  std::vector<double> opw;
+  WaveOps wops;
+  if (p->physics == DGLM_EULER && (p->precision == DGLM_FP64 || p->precision == DGLM_FP32) &&
+      (long long)K * Np < (1LL << 31))
+    wops = wave_ops(p->N);
+  if (wops.eb) wops.fill(op.data(), opw);
 
   // Tables of the fused mixed-precision Euler kernel (no Dirichlet faces:
   // those take the generic MFMA kernel).
@@ -806,9 +762,10 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
 
   // Visiting orders of the batches.
   std::vector<float> centroid = element_centroids(m, p->N, Np);
-  std::vector<int> ws_order, cols_order;
+  std::vector<int> wave_order, mx_order, cols_order;
   if (!centroid.empty()) {
-    if (!afr_ws.empty() || !mx_tab.empty()) ws_order = batch_order(centroid, 16);
+    if (wops.eb) wave_order = batch_order(centroid, wops.eb);
+    if (!mx_tab.empty()) mx_order = batch_order(centroid, 16);
     // (a small mesh is in the L2 whatever the order, and its stages are chains of
     // loads, of which the table would be one more)
     if (!cfr.empty() && (K + cops.eb - 1) / cops.eb > 2048) cols_order = batch_order(centroid, cops.eb);
@@ -824,6 +781,8 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
   c->nvar = p->physics == DGLM_EULER ? 5 : 1;
   c->dev = p->device;
   c->cols = cops;
+  c->wave = wops;
+  hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->dev);
   c->h_centroid.swap(centroid);
   c->nblk_ws = (K + wavespeed_elems(Np) - 1) / wavespeed_elems(Np);
   c->h_conn = conn;
@@ -849,9 +808,9 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
       (rc = dev_alloc(&c->conn, conn.size(), "conn")) || (rc = dev_alloc(&c->fmx, fmx.size(), "fmx")) ||
       (rc = dev_alloc(&c->clk, 2, "step clock")) ||
       (afrag_bytes && (rc = dev_alloc((char **)&c->afrag, afrag_bytes, "A-fragments"))) ||
-      (!afr_ws.empty() && (rc = dev_alloc(&c->afrag_ws, afr_ws.size(), "A-fragments (warp-specialised)"))) ||
-      (!arem_ws.empty() && (rc = dev_alloc(&c->arem_ws, arem_ws.size(), "remainder rows"))) ||
-      (!ws_order.empty() && (rc = dev_alloc(&c->ws_order, ws_order.size(), "batch order"))) ||
+      (!opw.empty() && (rc = dev_alloc(&c->op_wave, opw.size(), "operator"))) ||
+      (!wave_order.empty() && (rc = dev_alloc(&c->wave_order, wave_order.size(), "batch order"))) ||
+      (!mx_order.empty() && (rc = dev_alloc(&c->mx_order, mx_order.size(), "batch order"))) ||
       (!cfr.empty() && (rc = dev_alloc(&c->afrag_cols, cfr.size(), "operator streams"))) ||
       (!cols_order.empty() && (rc = dev_alloc(&c->cols_order, cols_order.size(), "batch order"))) ||
       (!rsum.empty() && (rc = dev_alloc(&c->rowsum, rsum.size(), "affine-offset tables"))) ||
@@ -885,11 +844,11 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
       hipMemcpy(c->conn, conn.data(), conn.size() * sizeof(int), hipMemcpyHostToDevice),
       hipMemcpy(c->fmx, fmx.data(), fmx.size() * sizeof(int), hipMemcpyHostToDevice),
       c->afrag ? hipMemcpy(c->afrag, afrag_src, afrag_bytes, hipMemcpyHostToDevice) : hipSuccess,
-      c->afrag_ws ? hipMemcpy(c->afrag_ws, afr_ws.data(), afr_ws.size() * sizeof(double), hipMemcpyHostToDevice)
-                  : hipSuccess,
-      c->arem_ws ? hipMemcpy(c->arem_ws, arem_ws.data(), arem_ws.size() * sizeof(double), hipMemcpyHostToDevice)
-                 : hipSuccess,
-      c->ws_order ? hipMemcpy(c->ws_order, ws_order.data(), ws_order.size() * sizeof(int), hipMemcpyHostToDevice)
+      c->op_wave ? hipMemcpy(c->op_wave, opw.data(), opw.size() * sizeof(double), hipMemcpyHostToDevice) : hipSuccess,
+      c->wave_order ? hipMemcpy(c->wave_order, wave_order.data(), wave_order.size() * sizeof(int),
+                                hipMemcpyHostToDevice)
+                    : hipSuccess,
+      c->mx_order ? hipMemcpy(c->mx_order, mx_order.data(), mx_order.size() * sizeof(int), hipMemcpyHostToDevice)
                   : hipSuccess,
       c->afrag_cols ? hipMemcpy(c->afrag_cols, cfr.data(), cfr.size() * sizeof(double), hipMemcpyHostToDevice)
                     : hipSuccess,
@@ -1297,9 +1256,9 @@ extern "C" int dglm_set_stage_kernel(dglm_ctx *c, int variant) {
   if (variant == DGLM_STAGE_MFMA_MX && !c->mx_tab)
     return fail(DGLM_ERR_UNSUPPORTED, "dglm_set_stage_kernel: the fused mixed-precision kernel is Euler with "
                                       "precision DGLM_FP32, N <= 6 and no Dirichlet faces");
-  if (variant == DGLM_STAGE_MFMA_WS && !c->afrag_ws)
+  if (variant == DGLM_STAGE_MFMA_WS && !c->op_wave)
     return fail(DGLM_ERR_UNSUPPORTED,
-                "dglm_set_stage_kernel: the warp-specialised kernel is Euler with N = 3 or 4 and precision "
+                "dglm_set_stage_kernel: the persistent kernel is Euler with N = 3 or 4 and precision "
                 "DGLM_FP64 or DGLM_FP32");
   if (variant == DGLM_STAGE_MFMA && !mfma_available(c->p.N))
     return fail(DGLM_ERR_UNSUPPORTED, "dglm_set_stage_kernel: no MFMA kernel for this order");

@@ -168,7 +168,7 @@ class Solver:
         """'auto', 'simple' (LDS-staged FP64; the packed-column kernel above
         N = 6), 'mfma' (FP64: packed columns; mixed precision: one workgroup
         per batch, operator rows in registers), 'mfma_ws' (persistent
-        warp-specialised FP64 Euler kernel, N = 3, 4) or 'mfma_mx' (fused
+        FP64 Euler kernel, a batch per wave, N = 3, 4) or 'mfma_mx' (fused
         mixed-precision Euler kernel)."""
         code = {"auto": A.DGLM_STAGE_AUTO, "simple": A.DGLM_STAGE_SIMPLE, "mfma": A.DGLM_STAGE_MFMA,
                 "mfma_ws": A.DGLM_STAGE_MFMA_WS, "mfma_mx": A.DGLM_STAGE_MFMA_MX}[variant]

@@ -40,7 +40,7 @@ enum { DGLM_ADVECTION = 0, DGLM_EULER = 1 };
  * three pieces and six products.  FP32 accumulation in all three.  Each
  * mode promises a result within its bound of FP64 (DGLM_FP32 and
  * DGLM_BF16X6 1e-8 relative), not a particular kernel: at Euler N = 3, 4
- * DGLM_FP32 runs the FP64 warp-specialised kernel, which is faster there than
+ * DGLM_FP32 runs the persistent FP64 kernel, which is faster there than
  * the mixed-precision one (dglm_set_stage_kernel(DGLM_STAGE_MFMA_MX) still
  * selects the latter). */
 enum { DGLM_FP64 = 0, DGLM_FP32 = 1, DGLM_BF16X3 = 2, DGLM_BF16X6 = 3 };
@@ -244,11 +244,10 @@ int dglm_set_timing(dglm_ctx *ctx, int on);
  * there); MFMA (N <= 6): in FP64 the packed-column kernel (every (variable,
  * element) pair of a batch a column of one MFMA contraction), in mixed precision
  * one workgroup per 16-element batch, operator row tiles in registers; MFMA_WS:
- * persistent warp-specialised FP64 Euler kernel (producer waves stage the next
- * batch while consumer waves run the MFMA contraction; N = 3, 4, precision
- * DGLM_FP64 or DGLM_FP32); MFMA_MX: fused mixed-precision Euler kernel
+ * persistent FP64 Euler kernel (operator in LDS, every wave on batches of its
+ * own; N = 3, 4, precision DGLM_FP64 or DGLM_FP32); MFMA_MX: fused mixed-precision Euler kernel
  * (DGLM_FP32, N <= 6, no Dirichlet faces).  AUTO in FP64 takes MFMA_WS for
- * Euler at N = 4 and K >= 20,480, else MFMA, else SIMPLE (N = 7..10); in mixed
+ * Euler at N = 3, 4 on meshes that fill its waves, else MFMA, else SIMPLE (N = 7..10); in mixed
  * precision MFMA_WS where it exists, else MFMA_MX, else MFMA.
  * dglm_get_stage_kernel reports the kernel that runs. */
 enum { DGLM_STAGE_AUTO = 0, DGLM_STAGE_SIMPLE = 1, DGLM_STAGE_MFMA = 2, DGLM_STAGE_MFMA_WS = 3, DGLM_STAGE_MFMA_MX = 4 };

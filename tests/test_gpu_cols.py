@@ -80,10 +80,10 @@ def test_ragged_element_counts(gpu, physics, N, K):
     _check(pb, physics, "lm", u, "mfma" if N <= 6 else None)
 
 
-@pytest.mark.parametrize("N,nhex,kernel", [(3, 3, "mfma"), (3, 16, "mfma"), (4, 12, "mfma"), (4, 16, "mfma_ws"),
-                                           (5, 3, "mfma"), (8, 2, "simple")])
+@pytest.mark.parametrize("N,nhex,kernel", [(3, 3, "mfma"), (3, 13, "mfma"), (3, 16, "mfma_ws"), (4, 11, "mfma"),
+                                           (4, 16, "mfma_ws"), (5, 3, "mfma"), (8, 2, "simple")])
 def test_kernel_chosen(gpu, N, nhex, kernel):
-    """FP64 Euler: the warp-specialised kernel only at N = 4 from five batches
-    per workgroup (K >= 20,480) on."""
+    """FP64 Euler: the persistent kernel only at N = 3, 4 on meshes that fill its
+    waves (2048, with 6 and 3 elements a round)."""
     with Solver(cube_problem(N, nhex), "euler") as s:
         assert s.stage_kernel() == kernel

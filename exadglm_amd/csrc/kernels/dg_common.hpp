@@ -85,6 +85,13 @@ __device__ inline bool step_dt(double t, double maxfs, double cfl_fac, double tm
   return true;
 }
 
+// Orders the compiler's LDS accesses of one wave; the LDS executes them in order.
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Raise the workgroup's part of maxfs to its largest x >= 0.  red: LDS, one
 // double per wave (at most 16 waves); every thread of the workgroup calls it.
 __device__ inline void raise_maxfs(DevClock *c, double x, double *red) {

@@ -198,9 +198,8 @@ __device__ inline void mx_surface_flux5(const double uM[5], const double uP[5], 
 
 // Cross-lane sums without the LDS crossbar: a double moved by one DPP
 // permutation (two 32-bit moves), and all-reduce sums over aligned groups of
-// 8 lanes (quad swaps, then the half-row mirror) and of 32 lanes (rotations
-// within a 16-lane row, then a swizzle with xor 16).  Every lane of a group
-// ends with the same sum, formed in a fixed order (deterministic).
+// 8 lanes (quad swaps, then the half-row mirror).  Every lane of a group ends
+// with the same sum, formed in a fixed order (deterministic).
 template <int CTRL>
 __device__ inline double dpp_f64(double x) {
   const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
@@ -219,13 +218,6 @@ __device__ inline double sum8(double x) {
   x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
   x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
   return x + dpp_f64<0x141>(x);  // row_half_mirror: the other quad of the 8
-}
-__device__ inline double sum32(double x) {
-  x += dpp_f64<0x128>(x);  // row_ror 8
-  x += dpp_f64<0x124>(x);  // row_ror 4
-  x += dpp_f64<0x122>(x);  // row_ror 2
-  x += dpp_f64<0x121>(x);  // row_ror 1
-  return x + swz_xor16_f64(x);
 }
 
 // Volume fluxes (fR, fS, fT) of variable v at one node: g_d . F with the
@@ -251,15 +243,45 @@ __device__ inline void mx_volume_flux1(int v, const double u[5], const double *g
   }
 }
 
+// Pressure and contravariant velocity of a volume pass's nodes, which do not
+// depend on the variable: formed once a batch and kept in registers, except at
+// N = 6, whose contraction waves have none left (the stage 672 us without them,
+// 696 to 704 with; N = 5 135 and 128, N = 2 57 and 54; K = 82,944 and 24,576).
+template <int N>
+struct MxNodes {
+  static constexpr int JX = (Ord<N>::Np + 31) / 32;
+  double V[JX][3], p[JX];
+  __device__ inline void form(int w, int lane, const double *s_u, const double *s_geo, double gamma) {
+    using S = MxShape<N>;
+    constexpr int EB = S::EB, UST = S::UST;
+    const int el = 2 * w + (lane >> 5), sl = lane & 31;
+    const double *gm = &s_geo[el * GEO_STRIDE];
+#pragma unroll
+    for (int x = 0; x < JX; x++) {
+      const int j = min(sl + 32 * x, S::Np - 1);
+      double u[5];
+#pragma unroll
+      for (int q = 0; q < 5; q++) u[q] = s_u[q * EB * UST + el * UST + j];
+      const double inv = rcp_refined(u[0]);
+      p[x] = (gamma - 1.0) * (u[4] - 0.5 * (u[1] * u[1] + u[2] * u[2] + u[3] * u[3]) * inv);
+      const double vx = u[1] * inv, vy = u[2] * inv, vz = u[3] * inv;
+#pragma unroll
+      for (int d = 0; d < 3; d++) V[x][d] = gm[3 * d] * vx + gm[3 * d + 1] * vy + gm[3 * d + 2] * vz;
+    }
+  }
+};
+
 // Volume pass of wave w for variable v: the volume fluxes at every node of
 // elements 2w, 2w+1 of the batch, their least-squares fits c (FP64, into cv)
 // and the FP32 remainders into vr [KV4][EB].  Lane (element el, group sl)
 // takes nodes j = sl + 32x; the fit sums meet across the 32 groups in
-// registers.  pv, vv: fit weights and basis as [q][Np] (a read of one q by
+// registers (twelve sums over all 32 lanes by five exchanges each were a third of
+// the pass: the stage 753 us at N = 6, K = 82,944, and 672 as below).  pv, vv: fit weights and basis as [q][Np] (a read of one q by
 // 32 consecutive nodes spreads over the LDS banks; [Np][4] put them on 8).
-template <int N>
-__device__ inline void mx_volume_pass(int v, int w, int lane, int ne, const double *s_u, const double *s_geo,
-                                      const double *pv, const double *vv, double gamma, double *cv, float *vr) {
+template <int N, bool KEPT>
+__device__ inline void mx_volume_pass(int v, int w, int lane, int ne, const MxNodes<N> &kept, const double *s_u,
+                                      const double *s_geo, const double *pv, const double *vv, double gamma,
+                                      double *cv, float *vr) {
   using S = MxShape<N>;
   constexpr int Np = S::Np, EB = S::EB, UST = S::UST, JX = (Np + 31) / 32;
   const int el = 2 * w + (lane >> 5), sl = lane & 31;
@@ -273,21 +295,49 @@ __device__ inline void mx_volume_pass(int v, int w, int lane, int ne, const doub
     const int j = sl + 32 * x;
     f[x][0] = f[x][1] = f[x][2] = 0.0;
     if (j < Np) {
-      double u[5];
+      const double *uj = &s_u[el * UST + j];
+      if constexpr (!KEPT) {
+        double u[5];
 #pragma unroll
-      for (int q = 0; q < 5; q++) u[q] = s_u[q * EB * UST + el * UST + j];
-      mx_volume_flux1(v, u, gm, gamma, f[x]);
+        for (int q = 0; q < 5; q++) u[q] = uj[q * EB * UST];
+        mx_volume_flux1(v, u, gm, gamma, f[x]);
+      } else if (v == 0) {
+        const double mx = uj[EB * UST], my = uj[2 * EB * UST], mz = uj[3 * EB * UST];
+#pragma unroll
+        for (int d = 0; d < 3; d++) f[x][d] = gm[3 * d] * mx + gm[3 * d + 1] * my + gm[3 * d + 2] * mz;
+      } else {
+        const double c = uj[v * EB * UST];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+          f[x][d] = v == 4 ? (c + kept.p[x]) * kept.V[x][d] : c * kept.V[x][d] + gm[3 * d + v - 1] * kept.p[x];
+      }
 #pragma unroll
       for (int d = 0; d < 3; d++)
 #pragma unroll
         for (int q = 0; q < 4; q++) c[d * 4 + q] += pv[q * Np + j] * f[x][d];
     }
   }
+  // The twelve sums over 32 lanes: each half of the lanes keeps six, each
+  // quarter three, so that every exchange halves the values left; then all
+  // twelve come back from LDS.
 #pragma unroll
-  for (int q = 0; q < 12; q++) c[q] = sum32(c[q]);
-  if (sl == 0)
+  for (int q = 0; q < 6; q++) {
+    const double send = sl & 16 ? c[q] : c[q + 6], keep = sl & 16 ? c[q + 6] : c[q];
+    c[q] = keep + swz_xor16_f64(send);
+  }
 #pragma unroll
-    for (int q = 0; q < 12; q++) cv[q * EB + el] = c[q];
+  for (int q = 0; q < 3; q++) {
+    const double send = sl & 8 ? c[q] : c[q + 3], keep = sl & 8 ? c[q + 3] : c[q];
+    c[q] = sum8(keep + dpp_f64<0x128>(send));  // row_ror 8: the other eight of the row
+  }
+  if ((sl & 7) == 0) {
+    const int q0 = (sl & 16 ? 6 : 0) + (sl & 8 ? 3 : 0);
+#pragma unroll
+    for (int q = 0; q < 3; q++) cv[(q0 + q) * EB + el] = c[q];
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int q = 0; q < 12; q++) c[q] = cv[q * EB + el];
 #pragma unroll
   for (int x = 0; x < JX; x++) {
     const int j = sl + 32 * x;
@@ -317,6 +367,7 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
   static_assert(S::NW * 2 == EB && RT <= S::NW, "a volume pass takes two elements per wave");
   static_assert(NT == 4 * EB * 8, "the surface pass takes a thread per (face, group of eight)");
   static_assert(S::NW > RT && EB * 4 <= 64, "a helper wave stages the connectivity");
+  constexpr bool KEEP = RT < 6;
   const float *afrag = (const float *)(tab + TB::afr_off);
   const double *avfrag = (const double *)(tab + TB::avf_off);
 
@@ -506,8 +557,9 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
     //      waves of faces 2 and 3 (4..7), whose exterior traces lie farther
     //      away in memory, finish the surface pass later ----
     if (w < 4) {
-      mx_volume_pass<N>(0, w, lane, ne, &s_u[0][0], s_geo, pv, vv, gamma, s_c[0], s_vr[0]);
-      mx_volume_pass<N>(0, w + 4, lane, ne, &s_u[0][0], s_geo, pv, vv, gamma, s_c[0], s_vr[0]);
+      const MxNodes<N> none{};
+      mx_volume_pass<N, KEEP>(0, w, lane, ne, none, &s_u[0][0], s_geo, pv, vv, gamma, s_c[0], s_vr[0]);
+      mx_volume_pass<N, KEEP>(0, w + 4, lane, ne, none, &s_u[0][0], s_geo, pv, vv, gamma, s_c[0], s_vr[0]);
     }
     mx_barrier();
   };
@@ -526,6 +578,8 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
       const int b = order ? order[bq] : bq;
       const int e0 = b * EB, ne = min(EB, K - e0);
       stage_in(e0, ne, true);
+      MxNodes<N> nd;
+      if constexpr (KEEP) nd.form(w, lane, &s_u[0][0], s_geo, gamma);
       // the next batch (after the last one, this one again: the fetches are
       // unconditional, so that no path carries their registers through the
       // volume passes)
@@ -533,9 +587,11 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
       const int e1 = bn * EB, ne1 = min(EB, K - e1);
 #pragma unroll 1
       for (int v = 0; v < 4; v++) {
-        mx_volume_pass<N>(v + 1, w, lane, ne, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1], s_vr[(v + 1) & 1]);
+        mx_volume_pass<N, KEEP>(v + 1, w, lane, ne, nd, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1],
+                                s_vr[(v + 1) & 1]);
         if constexpr (RT == 6)  // the slot of contraction wave w - 2 (see below)
-          mx_volume_pass<N>(v + 1, w - 2, lane, ne, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1], s_vr[(v + 1) & 1]);
+          mx_volume_pass<N, KEEP>(v + 1, w - 2, lane, ne, nd, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1],
+                                s_vr[(v + 1) & 1]);
         if (v == 0) fetch_conn(e1, ne1);
         mx_barrier();
       }
@@ -562,6 +618,8 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
     const int b = order ? order[bq] : bq;
     const int e0 = b * EB, ne = min(EB, K - e0);
     stage_in(e0, ne, false);
+    MxNodes<N> nd;
+    if constexpr (KEEP) nd.form(w, lane, &s_u[0][0], s_geo, gamma);
     // ---- 4. per variable: the contraction, the fit term, the update, then
     //      this wave's share of the next variable's volume pass ----
 #pragma unroll 1
@@ -639,7 +697,8 @@ __global__ __launch_bounds__(MxShape<N>::NT) void stage_mx_kernel(StageArgs a, c
       // waves 0 and 1, whose chains take the MFMA pipe first: the helpers, on
       // SIMDs 2 and 3, run their volume-pass slots in the variable loop)
       if (v < 4 && (RT != 6 || w < 4))
-        mx_volume_pass<N>(v + 1, w, lane, ne, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1], s_vr[(v + 1) & 1]);
+        mx_volume_pass<N, KEEP>(v + 1, w, lane, ne, nd, &s_u[0][0], s_geo, pv, vv, gamma, s_c[v + 1],
+                                s_vr[(v + 1) & 1]);
       mx_barrier();  // remainder tile of v + 1 complete; the tile of v is free
     }
   }

@@ -57,13 +57,6 @@ inline void wave_arrange(const double *opT /*[KD][Np]*/, double *out) {
       }
 }
 
-// Orders the compiler's LDS accesses of one wave; the LDS executes them in order.
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Global value at a byte offset from a wave-uniform address.  The address stays
 // in scalar registers: a use the compiler cannot see through keeps it from
 // adding the offset in vector registers, one instruction for every access.

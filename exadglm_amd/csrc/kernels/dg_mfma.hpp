@@ -302,6 +302,11 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   constexpr int NVEL = PHYS == PHYS_ADV ? 3 : 1;
   static_assert(PREC != PREC_F64, "FP64 runs in the packed-column kernel");
   constexpr bool BF = PREC == PREC_BF;
+  // Unrolling of the fit's contraction in the epilogue: whole, but at N = 4 in
+  // split BF16, where the loads it hoists keep a second workgroup off the CU (Euler
+  // K = 24,576 481 us whole, 316 by four; advection 104 and 70; N = 2 162 and 180,
+  // N = 3 180 and 203, N = 5 620 and 617, FP32 at N = 4 61 and 68).
+  constexpr int FITU = BF && N == 4 ? 4 : NBLK * 4;
   constexpr int KS16 = S::KS16;
 
   __shared__ double s_u[NV][EB * Np];
@@ -530,7 +535,7 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
             if (BF) rhs += (double)acl[r];
             // exact FP64 contraction of the fit: sum_b sum_q c_bq (A_b V_b)_q
             const double *av = &fitAV[(size_t)i * NBLK * 4];
-#pragma unroll
+#pragma unroll FITU
             for (int bq = 0; bq < NBLK * 4; bq++) rhs += s_c[bq * EB + e] * av[bq];
             const size_t gi = v * KNp + (size_t)(e0 + e) * Np + i;
             if (MODE == 1) {

@@ -337,8 +337,8 @@ def main():
     dof_stage = K * Np * nvar * 5 * args.steps
     value = dof_stage / wall
     # Stage-kernel time inside the timed region: the graph-replayed step time
-    # less the per-step wave-speed and dt kernels (their event-timed averages
-    # from the eager steps after it), over the 5 stages.  The eager steps'
+    # less the wave-speed kernel (its event-timed average from the eager
+    # steps after it), over the 5 stages.  The eager steps'
     # own per-launch stage average is reported beside it.
     st_ms, st_n = tm["stage"]
     st_eager_s = st_ms / st_n / 1e3
@@ -360,8 +360,8 @@ def main():
     roof["traffic"], roof["traffic_source"] = profiled_traffic(ksym, args)
     roof["kernel"] = ksym
     roof["avg_launch_us"] = st_avg_s * 1e6
-    roof["avg_launch_us_source"] = ("timed graph-replayed steps: (ms_per_step - wave-speed and dt kernel "
-                                    "averages) / 5 stages")
+    roof["avg_launch_us_source"] = ("timed graph-replayed steps: (ms_per_step - wave-speed kernel "
+                                    "average) / 5 stages")
     roof["avg_launch_us_eager_events"] = st_eager_s * 1e6
     roof["algorithmic_bytes_per_launch"] = B
     roof["contraction_flops_per_launch"] = F

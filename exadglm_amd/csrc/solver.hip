@@ -527,12 +527,11 @@ int timer_flush(dglm_ctx *c) {
 
 // ---------------------------------------------------------------------------
 // Allocation-free stepping (dglm_step_noalloc; no reference counterpart):
-// its device scratch -- the dt history and the wave-speed block maxima with
-// their face indices -- lives in this fixed array instead of buffers the
-// library allocates.  Each device holds its own copy until the process ends;
-// every call on one device shares it, so calls that overlap on one device
-// race.  Layout in doubles: [0, MAX_STEPS) dt history, [MAX_STEPS, +MAX_BLOCKS)
-// block maxima, then MAX_BLOCKS int32 face indices.
+// its device scratch, the dt history, lives in this fixed array instead of a
+// buffer the library allocates.  Each device holds its own copy until the
+// process ends; every call on one device shares it, so calls that overlap on one
+// device race.  In doubles: [0, MAX_STEPS) dt history; the rest is unused (the
+// size is the one the header states).
 // ---------------------------------------------------------------------------
 constexpr size_t NOALLOC_DOUBLES = (size_t)DGLM_NOALLOC_MAX_STEPS + DGLM_NOALLOC_MAX_BLOCKS + DGLM_NOALLOC_MAX_BLOCKS / 2;
 static_assert(NOALLOC_DOUBLES * sizeof(double) == DGLM_NOALLOC_SCRATCH_BYTES, "scratch size");

@@ -298,6 +298,7 @@ inline bool mfma_available(int N) { return N >= 1 && N <= 6; }
 //     20,250 58.4/53.6, 48,000 116/101, 196,608 464/362
 bool wave_fills(const dglm_ctx *c) {
   const long per_round = (long)(c->cus / 8 * 8) * c->wave.nw * c->wave.eb;
+  if (per_round == 0) return false;  // (the device did not say how many CUs it has)
   const long rounds = (c->K + per_round - 1) / per_round;
   return c->K > 6144 && 5L * c->K >= 4 * rounds * per_round;
 }

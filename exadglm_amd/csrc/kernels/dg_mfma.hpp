@@ -286,8 +286,23 @@ __device__ inline void volume_flux_v(int v, const double *const u[5], const doub
   f2 = g[6] * F + g[7] * G + g[8] * H;
 }
 
+// Whether the contraction of the fit in the epilogue goes in steps of four instead
+// of unrolled whole.  Whole at N = 4 in split BF16, the loads it hoists keep a
+// second workgroup off the CU (Euler 255 VGPRs, rolled 176): a loss once there are
+// more batches than CUs, a gain before (us per pass of five steps, whole / rolled,
+// by batches of 16 elements on 256 CUs):
+//   Euler      11 2156/2269   47 2097/2194   192 2361/2435   274 4190/2516   1029 11458/9100
+//   advection  11  465/520                   192  476/531    274  874/576     375   892/588
+// The other orders and FP32 are whole throughout (us per Euler stage at K =
+// 24,576, whole / rolled: split BF16 N = 2 162/180, N = 3 180/203, N = 5 620/617;
+// FP32 N = 4 61/68).
+template <int N, int PREC>
+constexpr bool mfma_rolls(int nbatch, int cus) {
+  return PREC == PREC_BF && N == 4 && nbatch > cus;
+}
+
 //   MODE 0: LSRK update; MODE 1: write the RHS only.
-template <int N, int PHYS, int MODE, int PREC>
+template <int N, int PHYS, int MODE, int PREC, bool ROLLED>
 __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs a, const void *__restrict__ afrag_v,
                                                                       const double *__restrict__ fit,
                                                                       int nbatch) {
@@ -302,11 +317,7 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   constexpr int NVEL = PHYS == PHYS_ADV ? 3 : 1;
   static_assert(PREC != PREC_F64, "FP64 runs in the packed-column kernel");
   constexpr bool BF = PREC == PREC_BF;
-  // Unrolling of the fit's contraction in the epilogue: whole, but at N = 4 in
-  // split BF16, where the loads it hoists keep a second workgroup off the CU (Euler
-  // K = 24,576 481 us whole, 316 by four; advection 104 and 70; N = 2 162 and 180,
-  // N = 3 180 and 203, N = 5 620 and 617, FP32 at N = 4 61 and 68).
-  constexpr int FITU = BF && N == 4 ? 4 : NBLK * 4;
+  constexpr int FITU = ROLLED ? 4 : NBLK * 4;
   constexpr int KS16 = S::KS16;
 
   __shared__ double s_u[NV][EB * Np];

@@ -343,20 +343,29 @@ void launch_mx(dglm_ctx *c, const StageArgs &a) {
   }
 }
 
-template <int N, int PHYS, int MODE, int PREC>
-void launch_mfma(dglm_ctx *c, const StageArgs &a) {
+template <int N, int PHYS, int MODE, int PREC, bool ROLLED>
+void launch_mfma_as(dglm_ctx *c, const StageArgs &a, int nbatch) {
   using S = MfmaShape<N>;
-  const int nbatch = (c->K + 15) / 16;
   if (c->mfma_grid == 0) {
-    int dev = 0, cus = 0, occ = 0;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_mfma_kernel<N, PHYS, 0, PREC>, S::NT, 0);
-    c->mfma_grid = (cus > 0 ? cus : 256) * (occ > 0 ? occ : 1);
+    int occ = 0;
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, stage_mfma_kernel<N, PHYS, 0, PREC, ROLLED>, S::NT, 0);
+    c->mfma_grid = (c->cus > 0 ? c->cus : 256) * (occ > 0 ? occ : 1);
   }
   const int grid = nbatch < c->mfma_grid ? nbatch : c->mfma_grid;
-  hipLaunchKernelGGL((stage_mfma_kernel<N, PHYS, MODE, PREC>), dim3(grid), dim3(S::NT), 0, c->stream, a,
+  hipLaunchKernelGGL((stage_mfma_kernel<N, PHYS, MODE, PREC, ROLLED>), dim3(grid), dim3(S::NT), 0, c->stream, a,
                      (const void *)c->afrag, c->rowsum, nbatch);
+}
+
+template <int N, int PHYS, int MODE, int PREC>
+void launch_mfma(dglm_ctx *c, const StageArgs &a) {
+  const int nbatch = (c->K + 15) / 16;
+  if constexpr (mfma_rolls<N, PREC>(1, 0)) {  // (an order that is rolled on some meshes)
+    if (mfma_rolls<N, PREC>(nbatch, c->cus)) {
+      launch_mfma_as<N, PHYS, MODE, PREC, true>(c, a, nbatch);
+      return;
+    }
+  }
+  launch_mfma_as<N, PHYS, MODE, PREC, false>(c, a, nbatch);
 }
 
 template <int N, int PHYS, int MODE>

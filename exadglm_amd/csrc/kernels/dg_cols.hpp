@@ -693,15 +693,19 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
     double lfs = 0.0;
     for (int f0 = 0; f0 < 4 * ne; f0 += NT / 4) {
       const int fi = f0 + (tid >> 2), e = fi >> 2, f = fi & 3;
-      double mv2 = 0.0, mc2 = 0.0;
+      double mv2 = 0.0, mc2 = 0.0, sum = 0.0;
       if (fi < 4 * ne) {
         for (int j = tid & 3; j < Nfp; j += 4) {
           const int o = e * NS + s_fmx[(f * 4 + 3) * Nfp + j];
           const double v2 = s_x[o], c2 = s_x[EB * NS + o];
           mv2 = v2 > mv2 ? v2 : mv2;
           mc2 = c2 > mc2 ? c2 : mc2;
+          sum += v2 + c2;
         }
       }
+      // (a state that is not a number reaches dt as an infinite wave speed: the
+      // maxima pass over a NaN, the sum of the squares does not)
+      if (sum != sum) lfs = INFINITY;
 #pragma unroll
       for (int q = 1; q <= 2; q <<= 1) {
         mv2 = fmax(mv2, __shfl_xor(mv2, q, 64));
@@ -710,10 +714,7 @@ __global__ __launch_bounds__(64 * NW, 2) void stage_cols_kernel(StageArgs a, con
       if (fi < 4 * ne && (tid & 3) == 0) {
         const double lam = sqrt(mv2) + sqrt(mc2);
         a.lam_out[(size_t)e0 * 4 + fi] = lam;
-        double x = lam * s_geo[e * GEO_STRIDE + 9 + f * 4 + 3];
-        // (a non-finite state reaches dt as an infinite wave speed)
-        if (x != x) x = INFINITY;
-        lfs = fmax(lfs, x);
+        lfs = fmax(lfs, lam * s_geo[e * GEO_STRIDE + 9 + f * 4 + 3]);
       }
     }
     raise_maxfs(a.clk_out, lfs, s_tau);

@@ -49,22 +49,25 @@ __global__ __launch_bounds__(256) void wavespeed_lds_kernel(int K, const double 
   double lfs = 0.0;
   if (tid < ne * 4) {
     const int e = tid >> 2, f = tid & 3;
-    double mv2 = 0.0, mc2 = 0.0;
+    double mv2 = 0.0, mc2 = 0.0, sum = 0.0;
     for (int j = 0; j < Nfp; j++) {
       const int q = e * Np + s_fm[f * Nfp + j];
       const double v2 = s_v2[q];
       mv2 = v2 > mv2 ? v2 : mv2;
+      sum += v2;
       if (PHYS == PHYS_EULER) {
         const double c2 = s_c2[q];
         mc2 = c2 > mc2 ? c2 : mc2;
+        sum += c2;
       }
     }
     const double lam = PHYS == PHYS_EULER ? sqrt(mv2) + sqrt(mc2) : sqrt(mv2);
     maxv[fid] = lam;
     lfs = lam * geo[(size_t)(e0 + e) * GEO_STRIDE + 9 + f * 4 + 3];
-    // A non-finite state (no maximum over a NaN) reaches dt as an infinite
-    // wave speed: dt = 0 is flagged as bad on the device.
-    if (lfs != lfs) lfs = INFINITY;
+    // A state that is not a number reaches dt as an infinite wave speed, and dt = 0
+    // is flagged as bad on the device.  The face maxima pass over a NaN, the sum of
+    // the squares (all >= 0) does not.
+    if (sum != sum) lfs = INFINITY;
   }
   if (clk) {
     raise_maxfs(clk, lfs, red);

@@ -92,9 +92,12 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Raise the workgroup's part of maxfs to its largest x >= 0.  red: LDS, one
-// double per wave (at most 16 waves); every thread of the workgroup calls it.
+// Raise the workgroup's part of maxfs to its largest x.  Nothing below 0 gets there
+// (Fscale of an inside-out element is negative, and a negative double's bits are
+// above every positive one's).  red: LDS, one double per wave (at most 16 waves);
+// every thread of the workgroup calls it.
 __device__ inline void raise_maxfs(DevClock *c, double x, double *red) {
+  x = fmax(x, 0.0);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;

@@ -868,9 +868,11 @@ extern "C" int dglm_create(const dglm_params *p, const dglm_mesh *m, dglm_ctx **
                 : hipSuccess,
       c->dmap ? hipMemcpy(c->dmap, dmap.data(), dmap.size() * sizeof(int), hipMemcpyHostToDevice) : hipSuccess,
       c->mx_tab ? hipMemcpy(c->mx_tab, mx_tab.data(), mx_tab.size(), hipMemcpyHostToDevice) : hipSuccess,
-      hipMemset(c->clk, 0, 2 * sizeof(DevClock)),
-      hipMemset(c->u[0], 0, nst * sizeof(double)),
-      hipMemset(c->u[1], 0, nst * sizeof(double)),
+      // (fills may return before they are done, and the context's stream does not
+      // wait for the null stream)
+      hipMemsetAsync(c->clk, 0, 2 * sizeof(DevClock), c->stream),
+      hipMemsetAsync(c->u[0], 0, nst * sizeof(double), c->stream),
+      hipMemsetAsync(c->u[1], 0, nst * sizeof(double), c->stream),
   };
   for (hipError_t e : errs)
     if (e != hipSuccess) {

@@ -16,8 +16,7 @@
 //   * the D-fragment is consumed in registers by the LSRK update
 //     k = a k + dt rhs, u_out = u_in + b k (FP64 in every precision).
 //
-// Precision modes (PREC_F64 names the v_mfma_f64_16x16x4f64 traits of the other
-// kernels; D register r of lane l is row 4r + l/16, column l%16):
+// Precision modes:
 //   PREC_F32  v_mfma_f32_16x16x4f32 on  B - c, where c is the least-squares
 //             affine fit of B over the nodes of each (element, variable,
 //             block) -- blocks are the three volume directions and the four
@@ -47,7 +46,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-enum { PREC_F64 = 0, PREC_F32 = 1, PREC_BF = 2 };
+enum { PREC_F32 = 1, PREC_BF = 2 };
 constexpr int BF_PIECES = 3;  // bf16 pieces kept per operand value (6-term product)
 
 // bf16 bits of x: round to nearest even of the FP32 value of x (finite x).
@@ -82,15 +81,6 @@ struct MfmaShape {
 
 template <int PREC>
 struct PrecTraits;
-template <>
-struct PrecTraits<PREC_F64> {
-  typedef double T;
-  typedef f64x4 Acc;
-  __device__ static inline Acc mfma(double a, double b, Acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline int row(int lane, int r) { return 4 * r + (lane >> 4); }
-};
 template <>
 struct PrecTraits<PREC_F32> {
   typedef float T;
@@ -315,7 +305,6 @@ __global__ __launch_bounds__(MfmaShape<N>::NT) void stage_mfma_kernel(StageArgs 
   constexpr int NV = NVar<PHYS>::value;
   constexpr int EB = 16;
   constexpr int NVEL = PHYS == PHYS_ADV ? 3 : 1;
-  static_assert(PREC != PREC_F64, "FP64 runs in the packed-column kernel");
   constexpr bool BF = PREC == PREC_BF;
   constexpr int FITU = ROLLED ? 4 : NBLK * 4;
   constexpr int KS16 = S::KS16;

@@ -152,9 +152,9 @@ __device__ inline void mx_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_ba
 // Surface flux of the five variables times Fscale at one face-node pair:
 // LM (the reference's, euler_dglm.cpp:110-183) or Rusanov.  g = (nx, ny, nz,
 // Fscale) of the face.
-// euler_normal_flux5 / euler_rusanov5 (dg_fp64.hpp) with rcp_refined and
-// sqrt_refined: the surface and volume passes are the critical paths of the
-// stage-in and the variable loop
+// The fluxes of all five variables with the primitives of a trace formed once,
+// by rcp_refined and sqrt_refined: the surface and volume passes are the critical
+// paths of the stage-in and the variable loop.
 __device__ inline void mx_normal_flux5(const double U[5], const double *n, double gamma, double F[5], double &lam) {
   const double inv = rcp_refined(U[0]);
   const double p = (gamma - 1.0) * (U[4] - 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) * inv);

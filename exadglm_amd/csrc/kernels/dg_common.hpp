@@ -15,13 +15,15 @@ struct Ord {
 };
 
 // Reciprocal and square root of the stage kernels (the adjoint's pass A, where
-// they were measured no faster, divides): the hardware estimates v_rcp_f64 and v_rsq_f64 refined by Newton steps (two
-// r += r (1 - x r); for the root a coupled step on g = x y, h = y / 2 and a
-// correction g += h (x - g^2)), within an ulp of the IEEE results and equal
-// to them on every one of 4M sampled densities in [1e-3, 1e3] and squared
-// sound speeds in [1e-6, 1e6]; the IEEE division and square-root sequences
-// are chains about twice as long.  For positive normal arguments (densities,
-// squared sound speeds); zero and NaN pass through the root.
+// they were measured no faster, divides): the hardware estimates v_rcp_f64 and
+// v_rsq_f64 refined by Newton steps (two r += r (1 - x r); for the root a coupled
+// step on g = x y, h = y / 2 and a correction g += h (x - g^2)), within an ulp of
+// the IEEE results and equal to them on every one of 4M sampled densities in
+// [1e-3, 1e3] and squared sound speeds in [1e-6, 1e6]; the IEEE division and
+// square-root sequences are chains about twice as long.  For normal arguments, as
+// a sound state has them.  The reciprocal of 0 or an infinity is NaN, where the
+// division has an infinity or 0, so the fluxes of a state with such a density are
+// NaN; zero and NaN pass through the root.
 __device__ inline double rcp_refined(double x) {
   double r = __builtin_amdgcn_rcp(x);
   double e = __builtin_fma(-x, r, 1.0);

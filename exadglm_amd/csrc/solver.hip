@@ -288,10 +288,11 @@ void launch_wavespeed(dglm_ctx *c, const double *u, double *maxv, DevClock *clk)
 inline bool mfma_available(int N) { return N >= 1 && N <= 6; }
 
 // Whether the persistent kernel (one wave per batch, dg_wave.hpp) is the faster
-// one on this FP64 mesh: its waves take batches in rounds, so the last round
-// should leave few of them idle, and below one round of order 4 the packed-column
-// kernel also leaves the next step's wave speeds.  Measured (us per stage, LM
-// flux, packed columns / persistent):
+// one on this FP64 mesh: its waves take batches in rounds, and over the rounds at
+// least four fifths of them should have one (a nearly empty last round counts the
+// less the more there are before it).  At order 4 a single round does not do: there
+// the packed-column kernel also leaves the next step's wave speeds.  Measured (us
+// per stage, LM flux, packed columns / persistent, 256 CUs):
 //   N = 3 (12,288 elements a round)   K = 6000 13.5/16.6, 10,368 19.5/18.2, 13,182
 //     22.1/26.7, 20,250 31.2/27.8, 48,000 54.7/49.8, 196,608 223/185
 //   N = 4 (6144 a round)   K = 7986 29.5/31.8, 10,368 35.8/32.9, 13,182 42.8/42.5,
@@ -300,7 +301,7 @@ bool wave_fills(const dglm_ctx *c) {
   const long per_round = (long)(c->cus / 8 * 8) * c->wave.nw * c->wave.eb;
   if (per_round == 0) return false;  // (the device did not say how many CUs it has)
   const long rounds = (c->K + per_round - 1) / per_round;
-  return c->K > 6144 && 5L * c->K >= 4 * rounds * per_round;
+  return 5L * c->K >= 4 * rounds * per_round && (rounds > 1 || c->p.N == 3);
 }
 
 // The stage kernel that runs: the request where it exists, else the best
@@ -540,8 +541,8 @@ int timer_flush(dglm_ctx *c) {
 // its device scratch, the dt history, lives in this fixed array instead of a
 // buffer the library allocates.  Each device holds its own copy until the
 // process ends; every call on one device shares it, so calls that overlap on one
-// device race.  In doubles: [0, MAX_STEPS) dt history; the rest is unused (the
-// size is the one the header states).
+// device race.  In doubles: [0, MAX_STEPS) dt history; the rest is reserved (the
+// header states the size, and the block limit that went with it).
 // ---------------------------------------------------------------------------
 constexpr size_t NOALLOC_DOUBLES = (size_t)DGLM_NOALLOC_MAX_STEPS + DGLM_NOALLOC_MAX_BLOCKS + DGLM_NOALLOC_MAX_BLOCKS / 2;
 static_assert(NOALLOC_DOUBLES * sizeof(double) == DGLM_NOALLOC_SCRATCH_BYTES, "scratch size");
@@ -1098,10 +1099,13 @@ extern "C" int dglm_rhs(dglm_ctx *c, const double *u, double *rhs, double *maxv,
 namespace {
 // Whether a step leaves the wave speeds of its new state: advection's are
 // constant, and the packed-column kernel's last Euler stage forms them on meshes
-// of few batches, where the separate kernel costs mostly its launch (a step at
-// N = 4, K = 384: 46 -> 39 us; N = 5, K = 1296: 70 -> 62).  On larger ones its two
-// barriers at the end of every workgroup cost more than the kernel (N = 3, K =
-// 44,574: 8 us a step more, N = 4, K = 11,520: 3).
+// of few batches, where the separate kernel costs mostly its launch.  On larger
+// ones the two barriers it adds to every workgroup cost what the kernel does.  Us
+// per step by batches, kernel / last stage:
+//   N = 1   512 30.0/27.9   1000 33.8/31.8   2197 43.8/42.0   4096 53.6/51.2   5832 64.6/62.6
+//   N = 3   250 34.5/30.6   1024 43.8/40.2   2000 60.7/56.7   3456 89.0/88.2   5488 124/125
+//   N = 4   250 43.0/37.1   1024 68.4/62.8   2000 115/111     3456 164/165     5488 234/236
+//   N = 6   512 155/151     1331 346/344     2197 518/516     4096 902/902     5832 1361/1366
 constexpr int LEAVE_SPEEDS_MAX_BATCHES = 2048;
 bool step_leaves_speeds(const dglm_ctx *c) {
   if (c->nvar == 1) return true;

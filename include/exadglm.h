@@ -206,8 +206,8 @@ int dglm_step(dglm_ctx *ctx, int nsteps, double *dt_hist);
  * tight serving loops, harnesses that forbid hipMalloc).  Advances nsteps like
  * dglm_step, with the same kernels and bitwise the same states and dt history
  * (dt_hist [nsteps], host, may be NULL), but calls no hipMalloc, hipFree or
- * allocating library routine: its device scratch -- the dt history, and room for
- * the wave-speed block maxima -- lives in a fixed array of the library
+ * allocating library routine: its device scratch -- the dt history, and room that
+ * is reserved -- lives in a fixed array of the library
  * (DGLM_NOALLOC_SCRATCH_BYTES on every device it runs on, held until the
  * process ends), and the steps are launched one kernel at a time (no graph,
  * no timing events).  nsteps > DGLM_NOALLOC_MAX_STEPS, or a mesh with more

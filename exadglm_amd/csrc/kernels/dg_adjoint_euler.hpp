@@ -32,9 +32,19 @@ struct EulAdjShape {
   static constexpr int Np = O::Np, Nfp = O::Nfp, NFF = O::NFF, KD = O::KD;
   static constexpr int G = (Np + 3) / 4, NS = 4 * (G | 1);  // k-steps; column stride of rbar and the state (dg_cols.hpp)
   static constexpr int U = (KD + 3) / 4, GS = 4 * (U | 1);  // row units of A^T; column stride of g
-  static constexpr int EB = N <= 4 ? 6 : (N <= 9 ? 3 : 2);
-  static constexpr int NW = N <= 7 ? 4 : 8, NT = 64 * NW;
-  static constexpr int WPE = N <= 6 ? 3 : 2;  // waves per SIMD (3: three workgroups a CU)
+  // Elements and waves.  At N = 1 six elements are 24 nodes and 72 slots, a third of
+  // four waves' threads at best, so there one wave takes eight elements (us per four
+  // steps recorded and swept back, [elements, waves], the last at four waves a SIMD
+  // and the others at three):
+  //   K        [6,4]   [6,1]  [10,1]   [8,1]   [8,1]
+  //   750        625     651     647     670     620
+  //   3072       690     721     722     735     685
+  //   16,464    1170     989     937     981     929
+  //   48,000    2653    1935    1965    1926    1846
+  //   444,528  20384   11540   11645   11442   10554   ([8,2] 12500, [16,1] 11937)
+  static constexpr int EB = N == 1 ? 8 : N <= 4 ? 6 : (N <= 9 ? 3 : 2);
+  static constexpr int NW = N == 1 ? 1 : N <= 7 ? 4 : 8, NT = 64 * NW;
+  static constexpr int WPE = N == 1 ? 4 : N <= 6 ? 3 : 2;  // waves per SIMD (3: three workgroups a CU)
   static constexpr int NC = 5 * EB, CT = (NC + 15) / 16;
   static constexpr int KB = (G + 1) / 2;  // blocks of two k-steps
   static constexpr ColRoles<NW> roles = cols_roles<U, CT, NW>();
